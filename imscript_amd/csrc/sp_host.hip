@@ -12,6 +12,7 @@
 #include "sp_internal.h"
 #include "sp_cg.h"
 #include "sp_tiles.h"
+#include "sp_stream.h"
 #include "sp_amle.h"
 #include "../../include/simpois_hip.h"
 
@@ -412,6 +413,17 @@ struct LevelPlan {
 	GsFlowInst *d_flow = nullptr;
 	int *d_flags = nullptr;
 	int flow_blocks = 0, epoch = 0;
+	// streaming sweeps of the tiled members (sp_stream.h); nt = 0: not used
+	struct {
+		int form = 0, op = 0, nt = 0, nbw = 0, blocks = 0, nprog = 0;
+		bool small = false;
+		spk::SsInst *d_inst = nullptr;
+		std::vector<spk::SsInst> inst;
+		spk::SsTask *d_tasks = nullptr;
+		spk::SsBlock *d_bw = nullptr;
+		unsigned *d_claim = nullptr, *d_mx = nullptr;
+		int *d_prog = nullptr;
+	} ss;
 	bool any_cg = false;
 	// FP32 CG of this level, built on first use and kept with the plan
 	struct {
@@ -607,8 +619,8 @@ static int gs_flow_build(Plan &pl, const LevelPlan &L, int var,
 	}
 	TRY(pl.upload(d_fi, fi));
 	TRY(pl.upload(d_flags, flags));
-	if (!pl.gs_claim) {
-		TRY(pl.alloc(&pl.gs_claim, 1));
+	if (!pl.gs_claim) TRY(pl.alloc(&pl.gs_claim, 1));
+	if (!pl.gs_err) {
 		TRY(pl.alloc(&pl.gs_err, 1));
 		HIPCHK(hipMemset(pl.gs_err, 0, sizeof(int)));
 		if (hipHostMalloc(&pl.h_gs_err, sizeof(int)) != hipSuccess)
@@ -631,6 +643,102 @@ static int gs_build(Plan &pl, LevelPlan &L, int var)
 	return SP_OK;
 }
 
+// Whether a level's tiled members can be swept by the streaming kernel, and
+// its data if so.  It takes radius 1 with a positive step (its coefficient
+// marks a known pixel by a negative zero) and planes whose skewed layout a
+// 32-bit byte offset reaches.
+// SIMPOIS_HIP_GS_SHAPE and SIMPOIS_HIP_GS_FLOW=0 ask for the tiles.
+static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
+{
+	auto &ss = L.ss;
+	const char *shape = getenv("SIMPOIS_HIP_GS_SHAPE");
+	if (pl.R != 1 || !(pl.teff > 0) || L.tiled.empty() || !g_gs_flow || (shape && *shape))
+		return SP_OK;
+	int tmax = 0;
+	for (int m : L.tiled) tmax = std::max(tmax, L.nsweep[m]);
+	ss.form = tmax <= 16 ? 1 : 0;
+	ss.op = has_f ? spk::SS_POISSON : spk::SS_LAPLACE;
+	const int K = spk::SS_FORMS[ss.form].K, KT = K * spk::SS_FORMS[ss.form].NW;
+	for (int m : L.tiled) {
+		const int w = L.sp[m].w, h = L.sp[m].h;
+		if (w < 4 || h < 4) return SP_OK;
+		if (4.0 * (spk::ss_bands(h) + 1) * spk::ss_band_floats(w, KT) >= 4.0e9) return SP_OK;
+	}
+	std::vector<spk::SsInst> in;
+	std::vector<spk::SsBlock> bw;
+	struct Key { int key; spk::SsTask t; };
+	std::vector<Key> tasks;
+	std::vector<size_t> prog_off;
+	size_t nprog = 0;
+	for (int m : L.tiled) {
+		const int w = L.sp[m].w, h = L.sp[m].h, T = L.nsweep[m];
+		spk::SsInst I{};
+		I.u = L.sp[m].u; I.c = L.sp[m].c;
+		I.w = w; I.h = h; I.T = T; I.t = pl.teff;
+		const size_t BS = spk::ss_band_floats(w, KT), nb = spk::ss_bands(h);
+		I.BS = (unsigned)BS;
+		I.pad = spk::ss_pad(KT);
+		I.U = spk::ss_steps(w, KT);
+		I.nslot = (h + KT) / 64 + 3;
+		TRY(pl.alloc(&I.A, (nb + 1) * BS));
+		TRY(pl.alloc(&I.C, (nb + 1) * BS));
+		spk::launch_ss_clear(ss.op, I.C, (nb + 1) * BS, nullptr);
+		TRY(pl.alloc(&I.bz, (size_t)2 * I.nslot * I.U * KT));
+		const int nT = (T + KT - 1) / KT, id = (int)in.size();
+		prog_off.push_back(nprog);
+		nprog += (size_t)nT * I.nslot * spk::SS_PS;
+		for (int tb = 0; tb < nT; tb++) {
+			const int k0 = tb * KT, nwa = (std::min(KT, T - k0) + K - 1) / K;
+			const int k1 = k0 + nwa * K - 1;
+			// in the order in which they can start: a band lags the one above
+			// by about 5 phases, a block of sweeps the one before by about 8
+			for (int J = k0 / 64; J <= (h - 1 + k1) / 64; J++)
+				tasks.push_back({5 * (J - k0 / 64) + 8 * tb, {id, tb, J}});
+		}
+		for (int jb = 0; jb < (int)nb; jb++)
+			for (int sb = 0; sb * 64 < w + 63; sb++) bw.push_back({id, jb, sb});
+		in.push_back(I);
+	}
+	if (nprog > 0x7fffffff || tasks.size() > 0x7fffffff) return SP_OK;
+	std::stable_sort(tasks.begin(), tasks.end(),
+			[](const Key &a, const Key &b) { return a.key < b.key; });
+	std::vector<spk::SsTask> tl;
+	for (const Key &k : tasks) tl.push_back(k.t);
+	TRY(pl.alloc(&ss.d_claim, 1));
+	TRY(pl.alloc(&ss.d_prog, nprog));
+	TRY(pl.alloc(&ss.d_mx, 2));
+	for (size_t k = 0; k < in.size(); k++) {
+		in[k].prog = ss.d_prog + prog_off[k];
+		in[k].mx = ss.d_mx;
+	}
+	TRY(pl.upload(&ss.d_inst, in));
+	TRY(pl.upload(&ss.d_tasks, tl));
+	TRY(pl.upload(&ss.d_bw, bw));
+	if (!pl.gs_err) {
+		TRY(pl.alloc(&pl.gs_err, 1));
+		HIPCHK(hipMemset(pl.gs_err, 0, sizeof(int)));
+		if (hipHostMalloc(&pl.h_gs_err, sizeof(int)) != hipSuccess)
+			return set_err(SP_ERR_NOMEM, "pinned host allocation of 4 bytes failed");
+	}
+	ss.inst = in;
+	ss.nprog = (int)nprog;
+	ss.small = pl.teff <= 0.25f && tmax <= 100000;
+	ss.nbw = (int)bw.size();
+	ss.blocks = spk::ss_blocks(ss.form, ss.op);
+	ss.nt = (int)tl.size();
+	return SP_OK;
+}
+
+static void ss_run(Plan &pl, LevelPlan &L, const spk::SsInst *d_inst, hipStream_t s)
+{
+	auto &ss = L.ss;
+	spk::launch_ss_reset(ss.d_claim, ss.d_prog, ss.nprog, ss.d_mx, 2, s);
+	spk::launch_ss_in(ss.op, d_inst, ss.d_bw, ss.nbw, s);
+	spk::launch_ss_run(ss.form, ss.op, ss.small, ss.d_tasks, ss.nt, ss.blocks, d_inst,
+			ss.d_claim, ss.d_mx, GS_FLOW_SPIN, pl.gs_err, s);
+	spk::launch_ss_out(ss.op, d_inst, ss.d_bw, ss.nbw, s);
+}
+
 // ---------------------------------------------------------- autotuner
 //
 // With sp_params.autotune set, the first sweep of a level whose members run
@@ -644,6 +752,7 @@ struct TuneRec {
 	std::vector<long> key;
 	int var;
 	std::vector<float> ms;   // per variant
+	float ss_ms;             // streaming sweeps (1e30: the level cannot take them)
 };
 static std::mutex g_tune_mu;
 static std::vector<TuneRec> g_tune;
@@ -677,7 +786,8 @@ static int gs_tune(Plan &pl, LevelPlan &L, hipStream_t s)
 		std::lock_guard<std::mutex> lk(g_tune_mu);
 		for (const TuneRec &r : g_tune)
 			if (r.key == key) {
-				if (r.var != L.gs_var) TRY(gs_build(pl, L, r.var));
+				if (r.ss_ms > r.ms[r.var]) L.ss.nt = 0;
+				if (!L.ss.nt && r.var != L.gs_var) TRY(gs_build(pl, L, r.var));
 				return SP_OK;
 			}
 	}
@@ -741,12 +851,32 @@ static int gs_tune(Plan &pl, LevelPlan &L, hipStream_t s)
 		ms[v] = t;
 		if (t < ms[best]) best = v;
 	}
+	float ss_ms = 1e30f;
+	if (rc == SP_OK && L.ss.nt) {
+		std::vector<spk::SsInst> si = L.ss.inst;
+		for (size_t k = 0; k < si.size(); k++) si[k].u = gi[L.tiled[k]].u;
+		spk::SsInst *d_si = nullptr;
+		rc = pl.upload(&d_si, si);
+		for (int rep = 0; rep < 2 && rc == SP_OK; rep++) {
+			for (int m : L.tiled)
+				(void)hipMemcpyAsync(gi[m].u, L.sp[m].u, (size_t)L.sp[m].w * L.sp[m].h * 4,
+						hipMemcpyDeviceToDevice, s);
+			(void)hipEventRecord(a, s);
+			ss_run(pl, L, d_si, s);
+			(void)hipEventRecord(b, s);
+			if (hipEventSynchronize(b) != hipSuccess)
+				rc = set_err(SP_ERR_HIP, "autotune run failed");
+			(void)hipEventElapsedTime(&ss_ms, a, b);
+		}
+	}
 	(void)hipEventDestroy(a);
 	(void)hipEventDestroy(b);
 	TRY(rc);
+	const bool stream = ss_ms <= ms[best];
+	if (!stream) L.ss.nt = 0;
 	if (best != L.gs_var) TRY(gs_build(pl, L, best));
 	std::lock_guard<std::mutex> lk(g_tune_mu);
-	g_tune.push_back({key, best, ms});
+	g_tune.push_back({key, best, ms, ss_ms});
 	return SP_OK;
 }
 
@@ -772,8 +902,13 @@ extern "C" int sp_autotune_report(char *buf, int cap)
 			sp_with_shape(R, v, [&](auto sh) {
 				using S = decltype(sh);
 				snprintf(line, sizeof line, "%s%s%dx%dx%d:%.3f", v ? "," : "",
-						v == r.var ? "*" : "", S::BI, S::BJ, S::BT, r.ms[v]);
+						v == r.var && r.ms[v] < r.ss_ms ? "*" : "", S::BI, S::BJ, S::BT, r.ms[v]);
 			});
+			out += line;
+		}
+		if (r.ss_ms < 1e30f) {
+			snprintf(line, sizeof line, ",%sstream:%.3f", r.ss_ms <= r.ms[r.var] ? "*" : "",
+					r.ss_ms);
 			out += line;
 		}
 		out += "\n";
@@ -942,7 +1077,8 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 		}
 		L.nsmall = (int)small.size();
 		TRY(pl.upload(&L.d_small, small));
-		TRY(gs_build(pl, L, gs_default_var(pl.R)));
+		TRY(ss_build(pl, L, has_f));
+		if (!L.ss.nt || P.autotune) TRY(gs_build(pl, L, gs_default_var(pl.R)));
 	}
 	// parent (finer) and coarse descriptors aligned with each level's members
 	for (int k = 0; k < nlev; k++) {
@@ -981,7 +1117,17 @@ static int run_gs(Plan &pl, LevelPlan &L, hipStream_t s)
 	else if (L.nsmall)
 		spk::launch_gs_small(pl.R, L.d_insts, L.d_small, L.nsmall, L.small_lds,
 				L.small_threads, s);
-	if (L.wf_off.size() > 1) {
+	if (L.ss.nt) {
+		// algorithmic bytes: as for the tiles, per block of sweeps
+		ProfScope pr("gs_tile", s);
+		ss_run(pl, L, L.ss.d_inst, s);
+		pl.gs_flow_used = true;
+		double px = 0;
+		const int KT = spk::SS_FORMS[L.ss.form].K * spk::SS_FORMS[L.ss.form].NW;
+		for (const spk::SsInst &I : L.ss.inst)
+			px += (double)((I.T + KT - 1) / KT) * I.w * I.h;
+		pr.add(4, 12.0 * px);
+	} else if (L.wf_off.size() > 1) {
 		// algorithmic bytes: per pass of BT sweeps, read u and the
 		// coefficient plane and write u once (12 B per pixel)
 		ProfScope pr(pl.R == 1 ? "gs_tile" : "gs_tile_r23", s);
