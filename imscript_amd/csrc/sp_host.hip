@@ -656,9 +656,14 @@ static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
 		return SP_OK;
 	int tmax = 0;
 	for (int m : L.tiled) tmax = std::max(tmax, L.nsweep[m]);
-	ss.form = tmax <= 16 ? 1 : 0;
+	// the default 10 sweeps fill one block of 5 wavefronts of 2, whose phases
+	// are short (1920 x 1080 x 3: 543 us, by 4 of 4 675, by 4 of 8 1067);
+	// from two such blocks on, 4 of 4 (512 x 512, 2000 sweeps: 2.2 ms, 2.8,
+	// 2.6; 4096 x 4096 x 3, 256: 7.3, 8.9, 7.2)
+	ss.form = tmax <= 20 ? 1 : 0;
 	ss.op = has_f ? spk::SS_POISSON : spk::SS_LAPLACE;
-	const int K = spk::SS_FORMS[ss.form].K, KT = K * spk::SS_FORMS[ss.form].NW;
+	int K, KT;
+	spk::ss_form_shape(ss.form, K, KT);
 	for (int m : L.tiled) {
 		const int w = L.sp[m].w, h = L.sp[m].h;
 		if (w < 4 || h < 4) return SP_OK;
@@ -699,14 +704,16 @@ static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
 			for (int sb = 0; sb * 64 < w + 63; sb++) bw.push_back({id, jb, sb});
 		in.push_back(I);
 	}
-	if (nprog > 0x7fffffff || tasks.size() > 0x7fffffff) return SP_OK;
+	if (nprog > 0x7ffffff0 || tasks.size() > 0x7fffffff) return SP_OK;
 	std::stable_sort(tasks.begin(), tasks.end(),
 			[](const Key &a, const Key &b) { return a.key < b.key; });
 	std::vector<spk::SsTask> tl;
 	for (const Key &k : tasks) tl.push_back(k.t);
-	TRY(pl.alloc(&ss.d_claim, 1));
-	TRY(pl.alloc(&ss.d_prog, nprog));
-	TRY(pl.alloc(&ss.d_mx, 2));
+	// progress words, claim counter and the level's largest values
+	TRY(pl.alloc(&ss.d_prog, nprog + 3));
+	HIPCHK(hipMemset(ss.d_prog, 0, (nprog + 3) * sizeof(int)));
+	ss.d_claim = (unsigned *)ss.d_prog + nprog;
+	ss.d_mx = ss.d_claim + 1;
 	for (size_t k = 0; k < in.size(); k++) {
 		in[k].prog = ss.d_prog + prog_off[k];
 		in[k].mx = ss.d_mx;
@@ -732,11 +739,10 @@ static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
 static void ss_run(Plan &pl, LevelPlan &L, const spk::SsInst *d_inst, hipStream_t s)
 {
 	auto &ss = L.ss;
-	spk::launch_ss_reset(ss.d_claim, ss.d_prog, ss.nprog, ss.d_mx, 2, s);
 	spk::launch_ss_in(ss.op, d_inst, ss.d_bw, ss.nbw, s);
 	spk::launch_ss_run(ss.form, ss.op, ss.small, ss.d_tasks, ss.nt, ss.blocks, d_inst,
 			ss.d_claim, ss.d_mx, GS_FLOW_SPIN, pl.gs_err, s);
-	spk::launch_ss_out(ss.op, d_inst, ss.d_bw, ss.nbw, s);
+	spk::launch_ss_out(ss.op, d_inst, ss.d_bw, ss.nbw, (unsigned *)ss.d_prog, ss.nprog + 3, s);
 }
 
 // ---------------------------------------------------------- autotuner
@@ -1123,10 +1129,11 @@ static int run_gs(Plan &pl, LevelPlan &L, hipStream_t s)
 		ss_run(pl, L, L.ss.d_inst, s);
 		pl.gs_flow_used = true;
 		double px = 0;
-		const int KT = spk::SS_FORMS[L.ss.form].K * spk::SS_FORMS[L.ss.form].NW;
+		int K, KT;
+		spk::ss_form_shape(L.ss.form, K, KT);
 		for (const spk::SsInst &I : L.ss.inst)
 			px += (double)((I.T + KT - 1) / KT) * I.w * I.h;
-		pr.add(4, 12.0 * px);
+		pr.add(3, 12.0 * px);
 	} else if (L.wf_off.size() > 1) {
 		// algorithmic bytes: per pass of BT sweeps, read u and the
 		// coefficient plane and write u once (12 B per pixel)

@@ -24,9 +24,16 @@ constexpr int SS_C = 8;    // steps per phase (between two barriers)
 constexpr int SS_PS = 32;  // words between two tasks' progress words
 
 // the compiled forms: K sweeps per wavefront, NW wavefronts of sweeps
-struct SsForm { int K, NW; };
-constexpr SsForm SS_FORMS[] = {{8, 4}, {5, 2}};
-constexpr int SS_NFORM = 2;
+template <int K_, int NW_> struct SsForm { static constexpr int K = K_, NW = NW_; };
+template <class F> inline void sp_with_form(int form, F &&f)
+{
+	if (form == 0) f(SsForm<4, 4>());
+	else f(SsForm<2, 5>());
+}
+inline void ss_form_shape(int form, int &K, int &KT)
+{
+	sp_with_form(form, [&](auto f) { K = f.K; KT = f.K * f.NW; });
+}
 
 // one plane.  The values u and the coefficients are laid out by bands of 64
 // rows and, inside a band, by sigma = i + j: pixel (i, j) at
@@ -58,8 +65,6 @@ inline int ss_bands(int h) { return (h + 63) / 64; }
 inline size_t ss_band_floats(int w, int KT) { return (size_t)64 * (w + 63 + 2 * ss_pad(KT)); }
 
 int ss_blocks(int form, int op);   // work-groups that can be resident
-void launch_ss_reset(unsigned *claim, int *prog, int nprog, unsigned *mx, int nmx,
-		hipStream_t s);
 void launch_ss_clear(int op, float *C, size_t n, hipStream_t s);
 void launch_ss_in(int op, const SsInst *in, const SsBlock *bw, int nb, hipStream_t s);
 // small: the step and the sweeps are such that values bounded by those the
@@ -67,6 +72,8 @@ void launch_ss_in(int op, const SsInst *in, const SsBlock *bw, int nb, hipStream
 void launch_ss_run(int form, int op, bool small, const SsTask *tasks, int nt, int blocks,
 		const SsInst *in, unsigned *claim, const unsigned *mx, int spin_max, int *err,
 		hipStream_t s);
-void launch_ss_out(int op, const SsInst *in, const SsBlock *bw, int nb, hipStream_t s);
+// also sets words[0, nwords) (the progress words, claim and mx) to 0
+void launch_ss_out(int op, const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
+		int nwords, hipStream_t s);
 
 } // namespace spk

@@ -9,11 +9,13 @@
 // hyperplanes plus a few microseconds per band and block of sweeps.
 //
 // Against the tiles (sp_gs.h, LDS values and a barrier per hyperplane step)
-// an update costs 11 vector instructions instead of 22 and 6 LDS accesses:
-// 4096 x 4096 x 3 and 256 sweeps 7.4 ms instead of 15, 1920 x 1080 x 3 and 10
-// sweeps 0.87 ms instead of 1.6, 512 x 512 and 2000 sweeps 3.9 ms instead of
-// 6 (finest levels).  Bound: vector issue where there are tasks enough, else
-// the phases (1.6 to 2.4 us) that a band waits for the one above it.
+// an update costs 11 vector instructions and its share of a step's LDS
+// accesses instead of 22 and 6: finest levels of 4096 x 4096 x 3 with 256
+// sweeps 6.9 ms instead of 15, of 1920 x 1080 x 3 with 10 sweeps 0.55 ms
+// instead of 1.6, of 512 x 512 with 2000 sweeps 2.2 ms instead of 6.  Bound:
+// vector issue where there are tasks enough (4096 x 4096 x 3), else the
+// phases of 1.0 (2 sweeps a wavefront) to 1.4 us (4) times the 10.5 of them
+// that a band starts after the one above it.
 #include <algorithm>
 #include <limits.h>
 #include <type_traits>
@@ -158,11 +160,10 @@ struct SsLds {
 	float *lout, *zout;
 };
 
-// SS_C steps from the coefficient row crow on.  cv: the coefficients of the next SS_D steps,
-// each replaced after its use by the one SS_D steps on (crow + its offset).
-constexpr int SS_D = 4;
+// SS_C steps from the coefficient row crow on.  cv: the coefficients of the next SS_C
+// steps, each replaced after its use by the one SS_C steps on (crow + its offset).
 template <int K, int OP, int FORM>
-static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_D][K],
+static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_C][K],
 		__amdgpu_buffer_rsrc_t cbuf, unsigned crow, const unsigned (&voff)[K], const SsLds &l,
 		int lane, float t)
 {
@@ -187,11 +188,11 @@ static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_D]
 #pragma unroll
 		for (int k = K - 1; k >= 0; k--) {
 			yn[k] = ss_update<OP, FORM>(k ? q.Z[k - 1] : q.Zm, k ? zn[k - 1] : zm,
-					k ? q.Y[k - 1] : q.Ym, q.Y[k], zn[k], cv[c % SS_D][k], t);
+					k ? q.Y[k - 1] : q.Ym, q.Y[k], zn[k], cv[c][k], t);
 		}
 #pragma unroll
 		for (int k = 0; k < K; k++) {
-			cv[c % SS_D][k] = ss_coef(cbuf, voff[k], crow + (c + SS_D) * 256);
+			cv[c][k] = ss_coef(cbuf, voff[k], crow + (c + SS_C) * 256);
 			q.Y[k] = yn[k];
 			q.Z[k] = zn[k];
 		}
@@ -212,21 +213,19 @@ static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_D]
 	}
 }
 
-// GEN: the level holds values that need SS_GENERAL.  Both forms are launched;
-// the one that the level's values do not call for ends at once.
-template <int K, int NW, int OP, bool GEN>
+template <int K, int NW, int OP>
 __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_ss_run(const SsTask *tasks, int nt,
 		const SsInst *insts, unsigned *claim, const unsigned *mx, int spin_max, int *err)
 {
 	constexpr int C = SS_C, KT = K * NW, KP = K <= 4 ? 4 : 8;
-	static_assert(C * K <= 64 && KT < 64 && 64 % C == 0, "phase shape");
+	static_assert(C * K <= 64 && KT < 64 && 64 % C == 0 && NW <= 8, "phase shape");
 	__shared__ __align__(16) float line[NW + 1][2][C][64];   // [w]: into wavefront w
 	__shared__ __align__(16) float zin[NW + 1][4][C][KP];    // [w + 1]: lane 0 of wavefront w
 	__shared__ __align__(16) float zo[NW][2][C][KP];         // lane 63 of wavefront w
 	__shared__ int s_k;
 	// values bounded by these stay far from overflow: with 0 < t <= 1/4 a sweep
 	// averages, and the data term adds at most t |c| (finite by the first test)
-	if (mx && GEN == (mx[0] < __float_as_uint(1e33f) && mx[1] < __float_as_uint(1e28f))) return;
+	const bool gen = !mx || !(mx[0] < __float_as_uint(1e33f) && mx[1] < __float_as_uint(1e28f));
 	const int lane = threadIdx.x & 63;
 	const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 	for (;;) {
@@ -260,7 +259,7 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 		};
 		if (wv < NW) {
 			SsState<K> st;
-			float cv[SS_D][K];
+			float cv[SS_C][K];
 			unsigned voff[K];
 			const int kw = k0 + wv * K, jrow = j0 + lane - kw;
 #pragma unroll
@@ -277,7 +276,7 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 			const bool rows = j0 - (kw + K - 1) >= 1 && j0 + 63 - kw <= H - 2;
 			if (wv < nwa) {
 #pragma unroll
-				for (int c = 0; c < SS_D; c++)
+				for (int c = 0; c < SS_C; c++)
 #pragma unroll
 					for (int k = 0; k < K; k++)
 						cv[c][k] = ss_coef(cbuf, voff[k], cbase + 256u * (unsigned)(gs * C + c));
@@ -296,7 +295,7 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 					ss_barrier();
 				}
 			};
-			if (GEN) {
+			if (gen) {
 				run(std::integral_constant<int, SS_GENERAL>(), 0, nph);
 			} else {
 				// phases [pa, pb) touch no cell beside the image's border: their
@@ -309,8 +308,8 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 				run(std::integral_constant<int, SS_EDGE>(), pb, nph);
 			}
 		} else if (wv == NW) {
-			// fetches for phases p + 3 and p + 4 while phases p and p + 1 run: a
-			// fetch takes longer than a phase
+			// fetches for phase p + 1 while phase p runs (two round trips to the
+			// coherent memory, about 0.3 us each, are less than a phase)
 			const ss_flag prog = (ss_flag)pprog;
 			const int jmaxp = tb ? (H - 1 + k0 - 1) / 64 : -1, jminp = tb ? (k0 - KT) / 64 : 0;
 			const bool up = q > 0, prev = tb > 0 && J <= jmaxp;
@@ -336,7 +335,7 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 			const float *A = pA;
 			const float *bz = pbz + ((ptrdiff_t)(tb & 1) * nslot + max(q - 1, 0)) * U * KT;
 			const int ec = lane / K, ek = lane - ec * K;
-			struct Regs { float lv[C], uv, zv[NW]; int fu, fp, fw; } ra, rb;
+			struct Regs { float lv[C], uv, zv[NW]; } r;
 			const unsigned zlane = 4u * ((ec < C ? ec : 0) * KT + ek);
 			// every call loads the same, from addresses that exist; commit
 			// puts fv where the value is no pixel's
@@ -387,51 +386,18 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 					for (int w = 0; w < NW; w++) zin[w + 1][p & 3][ec][ek] = zv[w];
 				}
 			};
-			// waits until the values of phase p are there; what the flags held
-			// two phases ago (r) usually tells
-			auto ready = [&](int p, const Regs &r) {
+			auto fetch = [&](int p) {
 				if (p >= nph) return;
-				const int nu = p + gs - gsu + 1, np = p + gs - gsp + NW, nw = p + 2 - 64 / C;
-				if (up && su < nu) {
-					su = max(su, ss_uni(r.fu));
-					ss_wait(pu, nu, su, spin_max, err);
-				}
-				if (prev && p < nch && sp < np) {
-					sp = max(sp, ss_uni(r.fp));
-					ss_wait(pp, np, sp, spin_max, err);
-				}
-				if (sw < nw) {
-					sw = max(sw, ss_uni(r.fw));
-					ss_wait(pw, nw, sw, spin_max, err);
-				}
+				if (up) ss_wait(pu, p + gs - gsu + 1, su, spin_max, err);
+				if (prev && p < nch) ss_wait(pp, p + gs - gsp + NW, sp, spin_max, err);
+				ss_wait(pw, p + 2 - 64 / C, sw, spin_max, err);
+				issue(p, r);
+				commit(p, r);
 			};
-			auto peek = [&](Regs &r) {
-				r.fu = ss_ld(pu);
-				r.fp = ss_ld(pp);
-				r.fw = ss_ld(pw);
-			};
-			ra.fu = ra.fp = ra.fw = rb.fu = rb.fp = rb.fw = 0;
-			ready(0, ra);
-			issue(0, ra);
-			commit(0, ra);
-			ready(1, ra);
-			issue(1, ra);
-			ready(2, rb);
-			issue(2, rb);
-			peek(ra);
-			peek(rb);
+			fetch(0);
 			ss_barrier();
-			for (int p = 0; p < nph; p += 2) {
-				commit(p + 1, ra);
-				ready(p + 3, ra);
-				issue(p + 3, ra);
-				peek(ra);
-				ss_barrier();
-				if (p + 1 >= nph) break;
-				commit(p + 2, rb);
-				ready(p + 4, rb);
-				issue(p + 4, rb);
-				peek(rb);
+			for (int p = 0; p < nph; p++) {
+				fetch(p + 1);
 				ss_barrier();
 			}
 		} else {
@@ -444,12 +410,7 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 			const bool jok = (unsigned)jr < (unsigned)H;
 			float *bz = pbz + ((ptrdiff_t)(tb & 1) * nslot + q) * U * KT;
 			const int ec = lane / K, ek = lane - ec * K;
-			// every call stores C + NW times (lanes without a value: where no
-			// value belongs), so that waiting for all but those is waiting for the
-			// call before
 			float *const A = pA;
-			const unsigned anone = 4 * lane;
-			const unsigned bnone = 4u * (U - 1) * KT;
 			const bool rows = j0 - k1 >= 0 && j0 + 63 - k1 <= H - 1;
 			const unsigned zlane = 4u * (ec * KT + ek);
 			auto out = [&](int p) {
@@ -461,27 +422,25 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 					float *a = A + (ptrdiff_t)(pad - 2 * k1 + s) * 64;
 #pragma unroll
 					for (int c = 0; c < C; c++) ss_st_b(a + c * 64, arow, lp[c * 64]);
-				} else {
-					const bool on = jok && pl >= 0 && pl < nch;
+				} else if (pl >= 0 && pl < nch) {
 #pragma unroll
 					for (int c = 0; c < C; c++) {
 						const int i = s + c - 2 * k1 - jr;
-						const unsigned a = arow + 256u * (unsigned)(pad - 2 * k1 + s + c);
-						ss_st_b(A, on && (unsigned)i < (unsigned)W ? a : anone, lp[c * 64]);
+						if (jok && (unsigned)i < (unsigned)W)
+							ss_st_b(A + (ptrdiff_t)(pad - 2 * k1 + s + c) * 64, arow, lp[c * 64]);
 					}
 				}
-				const float *zp = &zo[0][p & 1][ec < C ? ec : 0][ek];
+				if (down && ec < C) {
+					const float *zp = &zo[0][p & 1][ec][ek];
 #pragma unroll
-				for (int w = 0; w < NW; w++) {
-					const int pw = p - 1 - w;
-					const bool on = down && w < nwa && pw >= 0 && pw < nch;
-					ss_st_b(bz, on && ec < C ? zlane + 4u * (unsigned)(pw * C * KT + w * K) : bnone,
-							zp[w * 2 * C * KP]);
+					for (int w = 0; w < NW; w++) {
+						const int pw = p - 1 - w;
+						if (w < nwa && pw >= 0 && pw < nch)
+							ss_st_b(bz + (ptrdiff_t)pw * C * KT + w * K, zlane, zp[w * 2 * C * KP]);
+					}
 				}
-				static_assert(C + NW == 12 || C + NW == 10, "wait count");
-				if (C + NW == 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-				else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
-				if (lane == 0) ss_st(prog, p - 1);
+				asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+				if (lane == 0) ss_st(prog, p < nph ? p : INT_MAX);
 			};
 			ss_barrier();
 			for (int p = 0; p < nph; p++) {
@@ -489,19 +448,8 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 				ss_barrier();
 			}
 			out(nph);
-			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-			if (lane == 0) ss_st(prog, INT_MAX);
 		}
 	}
-}
-
-__global__ __launch_bounds__(256) void k_ss_reset(unsigned *claim, int *prog, int nprog,
-		unsigned *mx, int nmx)
-{
-	const int i = blockIdx.x * 256 + threadIdx.x;
-	if (i == 0) *claim = 0;
-	if (i < nprog) prog[i] = 0;
-	if (i < nmx) mx[i] = 0;
 }
 
 // the coefficients of known pixels everywhere (the cells outside the image
@@ -570,9 +518,13 @@ __global__ __launch_bounds__(256) void k_ss_in(const SsInst *insts, const SsBloc
 }
 
 // the swept pixels back to the image layout
+// (and the words of the next run's synchronisation back to 0)
 template <int OP>
-__global__ __launch_bounds__(256) void k_ss_out(const SsInst *insts, const SsBlock *bw)
+__global__ __launch_bounds__(256) void k_ss_out(const SsInst *insts, const SsBlock *bw,
+		unsigned *words, int nwords)
 {
+	for (int i = blockIdx.x * 256 + threadIdx.x; i < nwords; i += gridDim.x * 256) words[i] = 0;
+
 	__shared__ float su[64][65];
 	const SsBlock b = bw[blockIdx.x];
 	const SsInst in = insts[b.inst];
@@ -598,15 +550,13 @@ __global__ __launch_bounds__(256) void k_ss_out(const SsInst *insts, const SsBlo
 	}
 }
 
-template <bool GEN, class F> static void ss_with(int form, int op, F &&f)
+template <class F> static void ss_with(int form, int op, F &&f)
 {
-	if (form == 0) {
-		if (op == SS_LAPLACE) f(k_ss_run<8, 4, SS_LAPLACE, GEN>, 6 * 64);
-		else f(k_ss_run<8, 4, SS_POISSON, GEN>, 6 * 64);
-	} else {
-		if (op == SS_LAPLACE) f(k_ss_run<5, 2, SS_LAPLACE, GEN>, 4 * 64);
-		else f(k_ss_run<5, 2, SS_POISSON, GEN>, 4 * 64);
-	}
+	sp_with_form(form, [&](auto fm) {
+		constexpr int K = decltype(fm)::K, NW = decltype(fm)::NW;
+		if (op == SS_LAPLACE) f(k_ss_run<K, NW, SS_LAPLACE>, (NW + 2) * 64);
+		else f(k_ss_run<K, NW, SS_POISSON>, (NW + 2) * 64);
+	});
 }
 
 int ss_blocks(int form, int op)
@@ -622,16 +572,8 @@ int ss_blocks(int form, int op)
 			ncu = 256;
 		nb = std::min(nb, std::max(1, per) * ncu);
 	};
-	ss_with<false>(form, op, ask);
-	ss_with<true>(form, op, ask);
+	ss_with(form, op, ask);
 	return nb;
-}
-
-void launch_ss_reset(unsigned *claim, int *prog, int nprog, unsigned *mx, int nmx,
-		hipStream_t s)
-{
-	const int n = std::max(std::max(nprog, nmx), 1);
-	k_ss_reset<<<(n + 255) / 256, 256, 0, s>>>(claim, prog, nprog, mx, nmx);
 }
 
 void launch_ss_clear(int op, float *C, size_t n, hipStream_t s)
@@ -653,14 +595,14 @@ void launch_ss_run(int form, int op, bool small, const SsTask *tasks, int nt, in
 		k<<<std::min(nt, blocks), threads, 0, s>>>(tasks, nt, in, claim, small ? mx : nullptr,
 				spin_max, err);
 	};
-	if (small) ss_with<false>(form, op, run);
-	ss_with<true>(form, op, run);
+	ss_with(form, op, run);
 }
 
-void launch_ss_out(int op, const SsInst *in, const SsBlock *bw, int nb, hipStream_t s)
+void launch_ss_out(int op, const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
+		int nwords, hipStream_t s)
 {
-	if (op == SS_LAPLACE) k_ss_out<SS_LAPLACE><<<nb, 256, 0, s>>>(in, bw);
-	else k_ss_out<SS_POISSON><<<nb, 256, 0, s>>>(in, bw);
+	if (op == SS_LAPLACE) k_ss_out<SS_LAPLACE><<<nb, 256, 0, s>>>(in, bw, words, nwords);
+	else k_ss_out<SS_POISSON><<<nb, 256, 0, s>>>(in, bw, words, nwords);
 }
 
 } // namespace spk
