@@ -118,17 +118,77 @@ __global__ __launch_bounds__(HD_T) void k_heatd_step(float *__restrict__ out,
 // are, so r is never -0 and adding a zero product leaves it unchanged.  A
 // non-finite corner makes its product, and r, NaN.
 
+// A tile whose values are finite and below lim (so that no sum of its T steps
+// overflows; the host's choice) takes a short form: no corner can matter, the
+// leading 0 + N and the exact product -4 C fold into the additions, and the
+// west and east neighbours are operands of theirs (lane shifts): 7 vector
+// operations per cell instead of 14 and two LDS permutes.  4096 x 4096 x 3,
+// 100 steps: 2.1 ms instead of 3.4 (125 us per launch of 6 steps, 79 of them
+// the time a copy of the planes takes).
+
 constexpr int HT_R = 48;          // rows per wave tile
 constexpr int HT_WAVES = 4;       // wave tiles per block, stacked vertically
+
+// the value of the lane to the west / east; 0 (a halo cell, whose value no
+// kept pixel sees) at the wave's ends
+static __device__ __forceinline__ float hd_west(float v)
+{
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+static __device__ __forceinline__ float hd_east(float v)
+{
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+
+// element i of a row in scalar registers: the lane's offset stays 32 bits (at
+// least 32 rows in 2^31 pixels)
+static __device__ __forceinline__ float hd_load(const float *row, int i)
+{
+	unsigned o = 4u * (unsigned)i;
+	asm("" : "+v"(o));
+	return gload_b<float>(row, o);
+}
+static __device__ __forceinline__ void hd_store(float *row, int i, float v)
+{
+	unsigned o = 4u * (unsigned)i;
+	asm("" : "+v"(o));
+	gstore_b<float>(row, o, v);
+}
+
+// one step of a tile of small finite values; EDGE: its columns reach an image
+// border (lanes atl, atr)
+template <int T, bool EDGE>
+static __device__ __forceinline__ void heatd_tile_step(float (&v)[HT_R], bool atl, bool atr,
+		bool top, bool bot, float t)
+{
+	float u = v[0], c = v[0];
+#pragma unroll
+	for (int r = 0; r < HT_R; r++) {
+		const float d = r + 1 < HT_R ? v[r + 1] : c;
+		float n = u, so = d, cw = hd_west(c), ce = hd_east(c);
+		if (EDGE) { cw = atl ? c : cw; ce = atr ? c : ce; }
+		if (r == T && top) n = c;
+		if (r == HT_R - 1 - T && bot) so = c;
+		float q = n + cw;
+		q = __builtin_fmaf(-4.0f, c, q);
+		q = q + ce;
+		q = q + so;
+		v[r] = c + t * (q * 0.25f);
+		u = c;
+		c = d;
+	}
+}
 
 // grid: x = tile columns of all planes (tiles_x per plane), y = groups of
 // HT_WAVES tile rows
 template <int T>
-__global__ __launch_bounds__(64 * HT_WAVES) void k_heatd_multi(float *__restrict__ out,
-		const float *__restrict__ in, int w, int h, int tiles_x, int tiles_y, float t)
+__global__ __launch_bounds__(64 * HT_WAVES) __attribute__((amdgpu_waves_per_eu(4)))
+void k_heatd_multi(float *__restrict__ out,
+		const float *__restrict__ in, int w, int h, int tiles_x, int tiles_y, float t, float lim)
 {
 	constexpr int OW = 64 - 2 * T, OH = HT_R - 2 * T;
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int lane = threadIdx.x & 63;
+	const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 	const int ty = blockIdx.y * HT_WAVES + wave;
 	if (ty >= tiles_y) return;
 	const int l = blockIdx.x / tiles_x, tx = blockIdx.x - l * tiles_x;
@@ -142,7 +202,7 @@ __global__ __launch_bounds__(64 * HT_WAVES) void k_heatd_multi(float *__restrict
 	for (int r = 0; r < HT_R; r++) {
 		int gj = gj0 + r;
 		gj = gj < 0 ? 0 : gj >= h ? h - 1 : gj;
-		v[r] = x[(size_t)gj * w + ci];
+		v[r] = hd_load(x + (size_t)gj * w, ci);
 	}
 	// per-lane clamps wherever the tile's columns reach an image border
 	const bool atl = gi == 0, atr = gi == w - 1;
@@ -152,7 +212,15 @@ __global__ __launch_bounds__(64 * HT_WAVES) void k_heatd_multi(float *__restrict
 	// reach past the image does not clamp, so rows within T-1 of such a
 	// border are wrong there and are left to the first / last tile
 	const bool top = y0 == 0, bot = y0 == h - OH;
-	for (int k = 0; k < T; k++) {
+	bool big = false;
+#pragma unroll
+	for (int r = 0; r < HT_R; r++) big |= !(__builtin_fabsf(v[r]) < lim);
+	if (!__any(big)) {
+		if (edge_cols)
+			for (int k = 0; k < T; k++) heatd_tile_step<T, true>(v, atl, atr, top, bot, t);
+		else
+			for (int k = 0; k < T; k++) heatd_tile_step<T, false>(v, atl, atr, top, bot, t);
+	} else for (int k = 0; k < T; k++) {
 		// window of old values: rows r-1 (u), r (c), r+1 (d), each with its
 		// west / east neighbours
 		// the corners of row r are the west / east neighbours of rows r-1
@@ -184,6 +252,7 @@ __global__ __launch_bounds__(64 * HT_WAVES) void k_heatd_multi(float *__restrict
 			u = c; uf = cf;
 			c = d; cw = dw; ce = de; cf = df;
 			v[r] = nv;
+			__builtin_amdgcn_sched_barrier(0);   // few registers in flight
 		}
 	}
 	if (lane < T || lane >= 64 - T) return;
@@ -191,7 +260,7 @@ __global__ __launch_bounds__(64 * HT_WAVES) void k_heatd_multi(float *__restrict
 #pragma unroll
 	for (int r = T; r < HT_R - T; r++) {
 		const int gj = gj0 + r;
-		if (gj >= jlo && gj < jhi) y[(size_t)gj * w + gi] = v[r];
+		if (gj >= jlo && gj < jhi) hd_store(y + (size_t)gj * w, gi, v[r]);
 	}
 }
 
@@ -234,13 +303,13 @@ __global__ __launch_bounds__(64 * HT_WAVES) void k_heatd_multi_field(float *__re
 	const bool top = y0 == 0, bot = y0 == h - OH;
 	for (int k = 0; k < T; k++) {
 		float c = v[0];
-		float cw = __shfl_up(c, 1, 64), ce = __shfl_down(c, 1, 64);
+		float cw = hd_west(c), ce = hd_east(c);
 		if (edge_cols) { cw = atl ? c : cw; ce = atr ? c : ce; }
 		float u = c, uw = cw, ue = ce;
 #pragma unroll
 		for (int r = 0; r < HR; r++) {
 			const float d = r + 1 < HR ? v[r + 1] : c;
-			float dw = __shfl_up(d, 1, 64), de = __shfl_down(d, 1, 64);
+			float dw = hd_west(d), de = hd_east(d);
 			if (edge_cols) { dw = atl ? d : dw; de = atr ? d : de; }
 			float n = u, nw = uw, ne = ue, so = d, sw = dw, se = de;
 			if (r == T && top) { n = c; nw = cw; ne = ce; }
@@ -322,13 +391,17 @@ bool launch_heatd_multi(float *out, const float *in, int w, int h, int pd, int T
 		float t, hipStream_t s)
 {
 	if (T < 1 || T > heatd_multi_max() || !heatd_multi_fits(w, h, T, HT_R)) return false;
+	// a step multiplies the largest magnitude by at most 1 + 2|t|, and its
+	// sums stay below 8 times it (NaN or huge t: no tile takes the short form)
+	float lim = 1e36f;
+	for (int k = 0; k < T; k++) lim /= 1.0f + 2.0f * __builtin_fabsf(t);
 	auto go = [&](auto tc) {
 		constexpr int TT = decltype(tc)::value;
 		constexpr int OW = 64 - 2 * TT, OH = HT_R - 2 * TT;
 		const int tiles_x = (w + OW - 1) / OW, tiles_y = (h + OH - 1) / OH;
 		const dim3 grid(tiles_x * pd, (tiles_y + HT_WAVES - 1) / HT_WAVES);
 		k_heatd_multi<TT><<<grid, 64 * HT_WAVES, 0, s>>>(out, in, w, h, tiles_x,
-				tiles_y, t);
+				tiles_y, t, lim);
 	};
 	switch (T) {
 	case 1: go(std::integral_constant<int, 1>{}); break;
