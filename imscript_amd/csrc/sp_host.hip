@@ -386,6 +386,18 @@ struct PlaneIn {            // one plane of one image (device pointers)
 	float *out;
 };
 
+// streaming sweeps of some planes (sp_stream.h); nt = 0: not used
+struct SsRun {
+	int form = 0, op = 0, nt = 0, nbw = 0, blocks = 0, nprog = 0;
+	bool small = false;
+	spk::SsInst *d_inst = nullptr;
+	std::vector<spk::SsInst> inst;
+	spk::SsTask *d_tasks = nullptr;
+	spk::SsBlock *d_bw = nullptr;
+	unsigned *d_claim = nullptr, *d_mx = nullptr;
+	int *d_prog = nullptr;
+};
+
 struct LevelPlan {
 	std::vector<int> members;        // plane ids present at this level
 	std::vector<SpPlane> sp;         // their descriptors at this level
@@ -413,17 +425,7 @@ struct LevelPlan {
 	GsFlowInst *d_flow = nullptr;
 	int *d_flags = nullptr;
 	int flow_blocks = 0, epoch = 0;
-	// streaming sweeps of the tiled members (sp_stream.h); nt = 0: not used
-	struct {
-		int form = 0, op = 0, nt = 0, nbw = 0, blocks = 0, nprog = 0;
-		bool small = false;
-		spk::SsInst *d_inst = nullptr;
-		std::vector<spk::SsInst> inst;
-		spk::SsTask *d_tasks = nullptr;
-		spk::SsBlock *d_bw = nullptr;
-		unsigned *d_claim = nullptr, *d_mx = nullptr;
-		int *d_prog = nullptr;
-	} ss;
+	SsRun ss;                        // streaming sweeps of the tiled members
 	bool any_cg = false;
 	// FP32 CG of this level, built on first use and kept with the plan
 	struct {
@@ -643,43 +645,36 @@ static int gs_build(Plan &pl, LevelPlan &L, int var)
 	return SP_OK;
 }
 
-// Whether a level's tiled members can be swept by the streaming kernel, and
-// its data if so.  It takes radius 1 with a positive step (its coefficient
-// marks a known pixel by a negative zero) and planes whose skewed layout a
-// 32-bit byte offset reaches.
-// SIMPOIS_HIP_GS_SHAPE and SIMPOIS_HIP_GS_FLOW=0 ask for the tiles.
-static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
+// Whether planes (u, c, w, h, T and t of each set in `in`) can be swept by the
+// streaming kernel, and its data if so, in memory of pl.  It takes positive
+// steps (the coefficient marks a known pixel by a negative zero) and planes
+// whose skewed layout a 32-bit byte offset reaches.  SIMPOIS_HIP_GS_FLOW=0
+// asks for the tiles.
+static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op)
 {
-	auto &ss = L.ss;
-	const char *shape = getenv("SIMPOIS_HIP_GS_SHAPE");
-	if (pl.R != 1 || !(pl.teff > 0) || L.tiled.empty() || !g_gs_flow || (shape && *shape))
-		return SP_OK;
+	if (in.empty() || !g_gs_flow) return SP_OK;
 	int tmax = 0;
-	for (int m : L.tiled) tmax = std::max(tmax, L.nsweep[m]);
+	for (const spk::SsInst &I : in) tmax = std::max(tmax, I.T);
 	// the default 10 sweeps fill one block of 5 wavefronts of 2, whose phases
 	// are short (1920 x 1080 x 3: 543 us, by 4 of 4 675, by 4 of 8 1067);
 	// from two such blocks on, 4 of 4 (512 x 512, 2000 sweeps: 2.2 ms, 2.8,
 	// 2.6; 4096 x 4096 x 3, 256: 7.3, 8.9, 7.2)
 	ss.form = tmax <= 20 ? 1 : 0;
-	ss.op = has_f ? spk::SS_POISSON : spk::SS_LAPLACE;
+	ss.op = op;
 	int K, KT;
 	spk::ss_form_shape(ss.form, K, KT);
-	for (int m : L.tiled) {
-		const int w = L.sp[m].w, h = L.sp[m].h;
-		if (w < 4 || h < 4) return SP_OK;
-		if (4.0 * (spk::ss_bands(h) + 1) * spk::ss_band_floats(w, KT) >= 4.0e9) return SP_OK;
+	for (const spk::SsInst &I : in) {
+		if (I.w < 4 || I.h < 4 || !(I.t > 0)) return SP_OK;
+		if (4.0 * (spk::ss_bands(I.h) + 1) * spk::ss_band_floats(I.w, KT) >= 4.0e9) return SP_OK;
 	}
-	std::vector<spk::SsInst> in;
 	std::vector<spk::SsBlock> bw;
 	struct Key { int key; spk::SsTask t; };
 	std::vector<Key> tasks;
 	std::vector<size_t> prog_off;
 	size_t nprog = 0;
-	for (int m : L.tiled) {
-		const int w = L.sp[m].w, h = L.sp[m].h, T = L.nsweep[m];
-		spk::SsInst I{};
-		I.u = L.sp[m].u; I.c = L.sp[m].c;
-		I.w = w; I.h = h; I.T = T; I.t = pl.teff;
+	for (size_t id = 0; id < in.size(); id++) {
+		spk::SsInst &I = in[id];
+		const int w = I.w, h = I.h, T = I.T;
 		const size_t BS = spk::ss_band_floats(w, KT), nb = spk::ss_bands(h);
 		I.BS = (unsigned)BS;
 		I.pad = spk::ss_pad(KT);
@@ -689,7 +684,7 @@ static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
 		TRY(pl.alloc(&I.C, (nb + 1) * BS));
 		spk::launch_ss_clear(ss.op, I.C, (nb + 1) * BS, nullptr);
 		TRY(pl.alloc(&I.bz, (size_t)2 * I.nslot * I.U * KT));
-		const int nT = (T + KT - 1) / KT, id = (int)in.size();
+		const int nT = (T + KT - 1) / KT;
 		prog_off.push_back(nprog);
 		nprog += (size_t)nT * I.nslot * spk::SS_PS;
 		for (int tb = 0; tb < nT; tb++) {
@@ -698,11 +693,10 @@ static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
 			// in the order in which they can start: a band lags the one above
 			// by about 5 phases, a block of sweeps the one before by about 8
 			for (int J = k0 / 64; J <= (h - 1 + k1) / 64; J++)
-				tasks.push_back({5 * (J - k0 / 64) + 8 * tb, {id, tb, J}});
+				tasks.push_back({5 * (J - k0 / 64) + 8 * tb, {(int)id, tb, J}});
 		}
 		for (int jb = 0; jb < (int)nb; jb++)
-			for (int sb = 0; sb * 64 < w + 63; sb++) bw.push_back({id, jb, sb});
-		in.push_back(I);
+			for (int sb = 0; sb * 64 < w + 63; sb++) bw.push_back({(int)id, jb, sb});
 	}
 	if (nprog > 0x7ffffff0 || tasks.size() > 0x7fffffff) return SP_OK;
 	std::stable_sort(tasks.begin(), tasks.end(),
@@ -729,20 +723,37 @@ static int ss_build(Plan &pl, LevelPlan &L, bool has_f)
 	}
 	ss.inst = in;
 	ss.nprog = (int)nprog;
-	ss.small = pl.teff <= 0.25f && tmax <= 100000;
+	// values stay small in averages: AMLE's, and the sweeps' for t <= 1/4
+	ss.small = tmax <= 100000;
+	for (const spk::SsInst &I : in)
+		if (op != spk::SS_AMLE && !(I.t <= 0.25f)) ss.small = false;
 	ss.nbw = (int)bw.size();
 	ss.blocks = spk::ss_blocks(ss.form, ss.op);
 	ss.nt = (int)tl.size();
 	return SP_OK;
 }
 
-static void ss_run(Plan &pl, LevelPlan &L, const spk::SsInst *d_inst, hipStream_t s)
+static void ss_run(Plan &pl, const SsRun &ss, const spk::SsInst *d_inst, hipStream_t s)
 {
-	auto &ss = L.ss;
 	spk::launch_ss_in(ss.op, d_inst, ss.d_bw, ss.nbw, s);
 	spk::launch_ss_run(ss.form, ss.op, ss.small, ss.d_tasks, ss.nt, ss.blocks, d_inst,
 			ss.d_claim, ss.d_mx, GS_FLOW_SPIN, pl.gs_err, s);
-	spk::launch_ss_out(ss.op, d_inst, ss.d_bw, ss.nbw, (unsigned *)ss.d_prog, ss.nprog + 3, s);
+	spk::launch_ss_out(d_inst, ss.d_bw, ss.nbw, (unsigned *)ss.d_prog, ss.nprog + 3, s);
+}
+
+// a level's tiled members; SIMPOIS_HIP_GS_SHAPE asks for the tiles
+static int ss_level(Plan &pl, LevelPlan &L, bool has_f)
+{
+	const char *shape = getenv("SIMPOIS_HIP_GS_SHAPE");
+	if (pl.R != 1 || (shape && *shape)) return SP_OK;
+	std::vector<spk::SsInst> in;
+	for (int m : L.tiled) {
+		spk::SsInst I{};
+		I.u = L.sp[m].u; I.c = L.sp[m].c;
+		I.w = L.sp[m].w; I.h = L.sp[m].h; I.T = L.nsweep[m]; I.t = pl.teff;
+		in.push_back(I);
+	}
+	return ss_build(pl, L.ss, in, has_f ? spk::SS_POISSON : spk::SS_LAPLACE);
 }
 
 // ---------------------------------------------------------- autotuner
@@ -868,7 +879,7 @@ static int gs_tune(Plan &pl, LevelPlan &L, hipStream_t s)
 				(void)hipMemcpyAsync(gi[m].u, L.sp[m].u, (size_t)L.sp[m].w * L.sp[m].h * 4,
 						hipMemcpyDeviceToDevice, s);
 			(void)hipEventRecord(a, s);
-			ss_run(pl, L, d_si, s);
+			ss_run(pl, L.ss, d_si, s);
 			(void)hipEventRecord(b, s);
 			if (hipEventSynchronize(b) != hipSuccess)
 				rc = set_err(SP_ERR_HIP, "autotune run failed");
@@ -1083,7 +1094,7 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 		}
 		L.nsmall = (int)small.size();
 		TRY(pl.upload(&L.d_small, small));
-		TRY(ss_build(pl, L, has_f));
+		TRY(ss_level(pl, L, has_f));
 		if (!L.ss.nt || P.autotune) TRY(gs_build(pl, L, gs_default_var(pl.R)));
 	}
 	// parent (finer) and coarse descriptors aligned with each level's members
@@ -1126,7 +1137,7 @@ static int run_gs(Plan &pl, LevelPlan &L, hipStream_t s)
 	if (L.ss.nt) {
 		// algorithmic bytes: as for the tiles, per block of sweeps
 		ProfScope pr("gs_tile", s);
-		ss_run(pl, L, L.ss.d_inst, s);
+		ss_run(pl, L.ss, L.ss.d_inst, s);
 		pl.gs_flow_used = true;
 		double px = 0;
 		int K, KT;
@@ -2314,6 +2325,7 @@ struct AmleSched {
 	int *d_flags = nullptr;
 	int nblocks = 0, epoch = 0;
 	int ntiles = 0;
+	SsRun ss;                         // streaming sweeps (4 neighbours)
 };
 
 struct AmlePlan {
@@ -2346,6 +2358,24 @@ static int amle_build(AmlePlan &A, int T)
 	std::vector<GsTile> tiles;
 	AmleSched sc;
 	sc.T = T;
+	// the streaming sweeps, unless a tile shape is asked for; the output
+	// buffer's planes are bound by amle_bind
+	if (A.nn == 4 && !getenv("SIMPOIS_HIP_AMLE_VARIANT")) {
+		std::vector<spk::SsInst> in;
+		for (int l = 0; l < ninst; l++) {
+			spk::SsInst I{};
+			I.c = A.c + (size_t)A.w * A.h * (l % A.pd);
+			I.w = A.w; I.h = A.h; I.T = T; I.t = 1.0f;
+			in.push_back(I);
+		}
+		TRY(ss_build(A.mem, sc.ss, in, spk::SS_AMLE));
+		if (sc.ss.nt) {
+			sc.px = (long)ninst * T * A.w * A.h;
+			*A.mem.h_gs_err = 0;
+			A.sched.push_back(sc);
+			return SP_OK;
+		}
+	}
 	int bt = 0;
 	if (!amle_with_shape(A.R, A.var, [&](auto sh) {
 			using S = decltype(sh);
@@ -2374,8 +2404,8 @@ static int amle_build(AmlePlan &A, int T)
 			TRY(A.mem.upload(&sc.d_flags, flags));
 			sc.nblocks = std::min(sc.ntiles, spk::amle_flow_blocks(A.R, A.var,
 					A.nn == 4 && (A.w > 1 || A.h > 1)));
-			if (!A.mem.gs_claim) {
-				TRY(A.mem.alloc(&A.mem.gs_claim, 1));
+			if (!A.mem.gs_claim) TRY(A.mem.alloc(&A.mem.gs_claim, 1));
+			if (!A.mem.gs_err) {
 				TRY(A.mem.alloc(&A.mem.gs_err, 1));
 				HIPCHK(hipMemset(A.mem.gs_err, 0, sizeof(int)));
 				if (hipHostMalloc(&A.mem.h_gs_err, sizeof(int)) != hipSuccess)
@@ -2397,20 +2427,35 @@ static int amle_bind(AmlePlan &A, float *d_out, hipStream_t s)
 	if (A.u_for == d_out) return SP_OK;
 	const size_t n = (size_t)A.w * A.h;
 	std::vector<GsInst> in;
+	std::vector<spk::SsInst> si;
 	for (auto &sc : A.sched) {
+		for (size_t l = 0; l < sc.ss.inst.size(); l++) {
+			sc.ss.inst[l].u = (l < (size_t)A.pd ? d_out : A.tinf) + n * (l % A.pd);
+			si.push_back(sc.ss.inst[l]);
+		}
+		if (sc.ss.nt) continue;
 		for (int l = 0; l < A.pd; l++)
 			in.push_back({d_out + n * l, A.c + n * l, A.w, A.h, sc.T, 0.0f, nullptr});
 		if (A.trace)
 			for (int l = 0; l < A.pd; l++)
 				in.push_back({A.tinf + n * l, A.c + n * l, A.w, A.h, sc.T, 0.0f, nullptr});
 	}
-	TRY(A.mem.stage(in.size() * sizeof(GsInst)));
+	const size_t in_bytes = in.size() * sizeof(GsInst), si_bytes = si.size() * sizeof(si[0]);
+	TRY(A.mem.stage(in_bytes + si_bytes));
 	HIPCHK(hipStreamSynchronize(s));
-	memcpy(A.mem.h_stage, in.data(), in.size() * sizeof(GsInst));
-	size_t off = 0;
+	memcpy(A.mem.h_stage, si.data(), si_bytes);
+	memcpy((char *)A.mem.h_stage + si_bytes, in.data(), in_bytes);
+	size_t off = 0, soff = 0;
 	for (auto &sc : A.sched) {
+		if (sc.ss.nt) {
+			const size_t k = sc.ss.inst.size();
+			HIPCHK(hipMemcpyAsync(sc.ss.d_inst, (spk::SsInst *)A.mem.h_stage + soff,
+					k * sizeof(spk::SsInst), hipMemcpyHostToDevice, s));
+			soff += k;
+			continue;
+		}
 		const size_t k = (size_t)(A.trace ? 2 : 1) * A.pd;
-		HIPCHK(hipMemcpyAsync(sc.d_insts, (GsInst *)A.mem.h_stage + off,
+		HIPCHK(hipMemcpyAsync(sc.d_insts, (GsInst *)((char *)A.mem.h_stage + si_bytes) + off,
 				k * sizeof(GsInst), hipMemcpyHostToDevice, s));
 		off += k;
 	}
@@ -2425,6 +2470,15 @@ static int amle_sweeps(AmlePlan &A, int T, hipStream_t s)
 	if (!sc) return set_err(SP_ERR_ARG, "AMLE schedule for %d sweeps missing", T);
 	ProfScope ps("amle_tile", s);
 	const bool fast4 = A.nn == 4 && (A.w > 1 || A.h > 1);
+	if (sc->ss.nt) {
+		ss_run(A.mem, sc->ss, sc->ss.d_inst, s);
+		A.mem.gs_flow_used = true;
+		int K, KT;
+		spk::ss_form_shape(sc->ss.form, K, KT);
+		ps.add(3, 12.0 * (double)sc->px / std::min(sc->T, KT));
+		HIPCHK(hipGetLastError());
+		return SP_OK;
+	}
 	if (sc->d_flags && sc->epoch >= 0x7ffffffe) sc->d_flags = nullptr;   // flags exhausted
 	if (sc->d_flags) {
 		spk::launch_amle_flow(A.R, A.var, sc->d_tiles, sc->ntiles, sc->nblocks, sc->d_insts,

@@ -56,7 +56,7 @@ struct SsInst {
 struct SsTask { int inst, tb, J; };   // band J of the tb-th block of sweeps
 struct SsBlock { int inst, jb, sb; }; // 64 x 64 block of the skewed layout
 
-enum { SS_LAPLACE = 0, SS_POISSON = 1 };
+enum { SS_LAPLACE = 0, SS_POISSON = 1, SS_AMLE = 2 };   // SS_AMLE: 4 neighbours
 
 inline int ss_pad(int KT) { return 2 * (64 + KT) + 2 * SS_C + 8; }
 // the most steps of a band, its own and those the band below asks for
@@ -73,7 +73,7 @@ void launch_ss_run(int form, int op, bool small, const SsTask *tasks, int nt, in
 		const SsInst *in, unsigned *claim, const unsigned *mx, int spin_max, int *err,
 		hipStream_t s);
 // also sets words[0, nwords) (the progress words, claim and mx) to 0
-void launch_ss_out(int op, const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
+void launch_ss_out(const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
 		int nwords, hipStream_t s);
 
 } // namespace spk

@@ -24,7 +24,7 @@
 
 namespace spk {
 
-constexpr unsigned SS_KNOWN0 = 0x80000000u;   // Laplace: known pixel (holes hold t)
+constexpr unsigned SS_KNOWN0 = 0x80000000u;   // Laplace, AMLE: known pixel (holes hold t)
 
 static __device__ __forceinline__ float ss_nan() { return __uint_as_float(SP_QNAN_BITS); }
 
@@ -116,6 +116,47 @@ static __device__ __forceinline__ float ss_term(float v, float x)
 	return FORM == SS_EDGE ? __builtin_amdgcn_fmed3f(d, d, 0.0f) : d;
 }
 
+// AMLE of 4 neighbours (sp_amle.h): the mean of the first strict minimum and
+// maximum in the order E, S, W, N.  With finite values those are the plain
+// minimum and maximum, in which NaN cells outside the image drop out; only
+// where they are equal does the order show, in the sign of a zero: then the
+// result is the first neighbour in the image.  SS_GENERAL scans, from the
+// first neighbour by its place (column i, row j), since a pixel may be NaN.
+static __device__ __forceinline__ float ss_min3(float a, float b, float c)
+{
+	float r;
+	asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+	return r;
+}
+static __device__ __forceinline__ float ss_max3(float a, float b, float c)
+{
+	float r;
+	asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+	return r;
+}
+template <int FORM>
+static __device__ __forceinline__ float ss_amle(float x, float e, float so, float w, float n,
+		float c, int i, int j, int W, int H)
+{
+	float f = e, y;
+	if (FORM == SS_GENERAL) {
+		if (i + 1 >= W) f = j + 1 < H ? so : i > 0 ? w : n;
+		float mn = f, mx = f;
+		mn = so < mn ? so : mn;
+		mx = so > mx ? so : mx;
+		mn = w < mn ? w : mn;
+		mx = w > mx ? w : mx;
+		mn = n < mn ? n : mn;
+		mx = n > mx ? n : mx;
+		y = (mn + mx) * 0.5f;
+	} else {
+		const float mn = ss_min3(ss_min3(e, so, w), n, n), mx = ss_max3(ss_max3(e, so, w), n, n);
+		if (FORM == SS_EDGE) f = e == e ? e : so == so ? so : w;
+		y = mn == mx ? f : (mn + mx) * 0.5f;
+	}
+	return __float_as_int(c) < 0 ? x : y;
+}
+
 template <int OP, int FORM>
 static __device__ __forceinline__ float ss_update(float x, float e, float so, float w,
 		float n, float c, float t)
@@ -165,7 +206,7 @@ struct SsLds {
 template <int K, int OP, int FORM>
 static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_C][K],
 		__amdgpu_buffer_rsrc_t cbuf, unsigned crow, const unsigned (&voff)[K], const SsLds &l,
-		int lane, float t)
+		int lane, float t, int i0, int jrow, int W, int H)
 {
 	constexpr int KP = K <= 4 ? 4 : 8;
 	float zi[K], zm, ym;
@@ -187,7 +228,11 @@ static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_C]
 		for (int k = 0; k < K; k++) zn[k] = ss_shift(zi[k], q.Y[k]);
 #pragma unroll
 		for (int k = K - 1; k >= 0; k--) {
-			yn[k] = ss_update<OP, FORM>(k ? q.Z[k - 1] : q.Zm, k ? zn[k - 1] : zm,
+			if (OP == SS_AMLE)
+				yn[k] = ss_amle<FORM>(k ? q.Z[k - 1] : q.Zm, k ? zn[k - 1] : zm,
+						k ? q.Y[k - 1] : q.Ym, q.Y[k], zn[k], cv[c][k], i0 + c - k,
+						jrow - k, W, H);
+			else yn[k] = ss_update<OP, FORM>(k ? q.Z[k - 1] : q.Zm, k ? zn[k - 1] : zm,
 					k ? q.Y[k - 1] : q.Ym, q.Y[k], zn[k], cv[c][k], t);
 		}
 #pragma unroll
@@ -289,8 +334,10 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 						const SsLds l = {&line[wv][p & 1][0][0], &zin[wv + 1][p & 3][0][0],
 							&zin[wv][(wv ? p - 1 : p) & 3][0][0],
 							&line[wv + 1][(p + 1) & 1][0][0], &zo[wv][(p + 1) & 1][0][0]};
+						const int s0 = (gs + p - wv) * C;
 						ss_chunk<K, OP, decltype(form)::value>(st, cv, cbuf,
-								cbase + 256u * (unsigned)((gs + p - wv) * C), voff, l, lane, t);
+								cbase + 256u * (unsigned)s0, voff, l, lane, t,
+								s0 - jrow - 2 * kw, jrow, W, H);
 					}
 					ss_barrier();
 				}
@@ -489,7 +536,7 @@ __global__ __launch_bounds__(256) void k_ss_in(const SsInst *insts, const SsBloc
 			if (!known) a1 = max(a1, sp_bits(cv[r]) & 0x7fffffffu);
 		}
 		su[jr][lane] = uv[r];
-		sc[jr][lane] = OP == SS_LAPLACE ? (known ? __uint_as_float(SS_KNOWN0) : in.t) : cv[r];
+		sc[jr][lane] = OP != SS_POISSON ? (known ? __uint_as_float(SS_KNOWN0) : in.t) : cv[r];
 	}
 #pragma unroll
 	for (int o = 32; o; o >>= 1) {
@@ -519,7 +566,6 @@ __global__ __launch_bounds__(256) void k_ss_in(const SsInst *insts, const SsBloc
 
 // the swept pixels back to the image layout
 // (and the words of the next run's synchronisation back to 0)
-template <int OP>
 __global__ __launch_bounds__(256) void k_ss_out(const SsInst *insts, const SsBlock *bw,
 		unsigned *words, int nwords)
 {
@@ -555,6 +601,7 @@ template <class F> static void ss_with(int form, int op, F &&f)
 	sp_with_form(form, [&](auto fm) {
 		constexpr int K = decltype(fm)::K, NW = decltype(fm)::NW;
 		if (op == SS_LAPLACE) f(k_ss_run<K, NW, SS_LAPLACE>, (NW + 2) * 64);
+		else if (op == SS_AMLE) f(k_ss_run<K, NW, SS_AMLE>, (NW + 2) * 64);
 		else f(k_ss_run<K, NW, SS_POISSON>, (NW + 2) * 64);
 	});
 }
@@ -578,12 +625,12 @@ int ss_blocks(int form, int op)
 
 void launch_ss_clear(int op, float *C, size_t n, hipStream_t s)
 {
-	k_ss_clear<<<1024, 256, 0, s>>>(C, n, sp_float(op == SS_LAPLACE ? SS_KNOWN0 : SP_KNOWN_BITS));
+	k_ss_clear<<<1024, 256, 0, s>>>(C, n, sp_float(op == SS_POISSON ? SP_KNOWN_BITS : SS_KNOWN0));
 }
 
 void launch_ss_in(int op, const SsInst *in, const SsBlock *bw, int nb, hipStream_t s)
 {
-	if (op == SS_LAPLACE) k_ss_in<SS_LAPLACE><<<nb, 256, 0, s>>>(in, bw);
+	if (op != SS_POISSON) k_ss_in<SS_LAPLACE><<<nb, 256, 0, s>>>(in, bw);
 	else k_ss_in<SS_POISSON><<<nb, 256, 0, s>>>(in, bw);
 }
 
@@ -598,11 +645,10 @@ void launch_ss_run(int form, int op, bool small, const SsTask *tasks, int nt, in
 	ss_with(form, op, run);
 }
 
-void launch_ss_out(int op, const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
+void launch_ss_out(const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
 		int nwords, hipStream_t s)
 {
-	if (op == SS_LAPLACE) k_ss_out<SS_LAPLACE><<<nb, 256, 0, s>>>(in, bw, words, nwords);
-	else k_ss_out<SS_POISSON><<<nb, 256, 0, s>>>(in, bw, words, nwords);
+	k_ss_out<<<nb, 256, 0, s>>>(in, bw, words, nwords);
 }
 
 } // namespace spk
