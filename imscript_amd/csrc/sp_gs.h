@@ -40,6 +40,8 @@ struct GsInst {
 	int w, h, nsweep;
 	float t;
 	const int *active;   // optional per-instance flag (nullptr = always on)
+	float *acc;          // where the values of the first sweeps are added up
+	                     // (k_gs_diag's and the streaming sweeps' summing forms)
 };
 
 // Skewed temporal tile: (instance, I', J', T').

@@ -97,7 +97,8 @@ static int g_dev_checked = 0, g_dev_ok = 0, g_max_lds = 65536;
 // SIMPOIS_HIP_GS_CELLS=0 turns it off (such levels then go to k_gs_small
 // or to tiles)
 static int g_gsc_lds = 0;
-static constexpr int GSC_LDS_MAX = 155000;
+static int g_gsd_lds = 0;   // the same of the kernel by diagonal
+static constexpr int GSC_LDS_MAX = 155000, GSD_LDS_MAX = 146000;
 static const int g_gsc_off = [] {
 	const char *e = getenv("SIMPOIS_HIP_GS_CELLS");
 	return e && !strcmp(e, "0") ? 1 : 0;
@@ -244,6 +245,7 @@ static int ensure_device()
 		g_max_lds = std::min(lds, 65536);
 	if (!g_gsc_off)
 		g_gsc_lds = spk::gs_cells_enable(GSC_LDS_MAX) == 0 ? GSC_LDS_MAX : g_max_lds;
+	if (!g_gsc_off) g_gsd_lds = spk::gs_diag_enable(GSD_LDS_MAX) == 0 ? GSD_LDS_MAX : 0;
 	(void)hipGetLastError();
 	g_dev_ok = 1;
 	return SP_OK;
@@ -389,7 +391,7 @@ struct PlaneIn {            // one plane of one image (device pointers)
 // streaming sweeps of some planes (sp_stream.h); nt = 0: not used
 struct SsRun {
 	int form = 0, op = 0, nt = 0, nbw = 0, blocks = 0, nprog = 0;
-	bool small = false;
+	bool small = false, sum = false;
 	spk::SsInst *d_inst = nullptr;
 	std::vector<spk::SsInst> inst;
 	spk::SsTask *d_tasks = nullptr;
@@ -419,6 +421,10 @@ struct LevelPlan {
 	long tile_pass_px = 0;           // for the profiler
 	int *d_small = nullptr;
 	int nsmall = 0, small_lds = 0, small_threads = 64;
+	// members swept by diagonal (k_gs_diag)
+	int *d_diag = nullptr;
+	int ndiag = 0, diag_lds = 0, diag_threads = 64;
+	bool diag_fdat = false;
 	int cells_slots = 0;             // slots per thread of k_gs_cells (0: k_gs_small)
 	// dependence-ordered tiles (k_gs_flow): member tile grids, one flag per
 	// grid cell, resident work-groups, flag value of the last launch
@@ -494,6 +500,9 @@ struct Plan {
 	int *gs_err = nullptr, *h_gs_err = nullptr;
 	bool gs_flow_used = false;
 
+	// where each plane's values after the first sweeps are added up (the
+	// adjoint's sweeps, one level without data terms); empty: not asked for
+	std::vector<float *> acc;
 	int transpose = 0;               // the CG applies the transposed biharmonic
 	                                 // operator (the adjoint's solve)
 	std::vector<char> key;           // identity of the call this plan serves
@@ -650,22 +659,30 @@ static int gs_build(Plan &pl, LevelPlan &L, int var)
 // steps (the coefficient marks a known pixel by a negative zero) and planes
 // whose skewed layout a 32-bit byte offset reaches.  SIMPOIS_HIP_GS_FLOW=0
 // asks for the tiles.
-static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op)
+static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bool sum = false)
 {
 	if (in.empty() || !g_gs_flow) return SP_OK;
 	int tmax = 0;
-	for (const spk::SsInst &I : in) tmax = std::max(tmax, I.T);
+	double px = 0;
+	for (const spk::SsInst &I : in) {
+		tmax = std::max(tmax, I.T);
+		px += (double)I.w * I.h;
+	}
 	// the default 10 sweeps fill one block of 5 wavefronts of 2, whose phases
 	// are short (1920 x 1080 x 3: 543 us, by 4 of 4 675, by 4 of 8 1067);
-	// from two such blocks on, 4 of 4 (512 x 512, 2000 sweeps: 2.2 ms, 2.8,
-	// 2.6; 4096 x 4096 x 3, 256: 7.3, 8.9, 7.2)
-	ss.form = tmax <= 20 ? 1 : 0;
+	// where the tasks wait for each other more than for the vector units, the
+	// short phases also pay for more blocks of sweeps (AMLE of 1500 x 2500, 80
+	// sweeps: 892 us, by 4 of 4 1035; 1024 x 1024, 100: 513 and 556), else not
+	// (512 x 512, 2000: 2.8 ms and 2.2; 4096 x 4096 x 3, 64: 3.2 and 2.9)
+	ss.form = tmax <= 20 || (tmax <= 128 && px * tmax < 2e9) ? 1 : 0;
 	ss.op = op;
+	ss.sum = sum;
 	int K, KT;
 	spk::ss_form_shape(ss.form, K, KT);
 	for (const spk::SsInst &I : in) {
 		if (I.w < 4 || I.h < 4 || !(I.t > 0)) return SP_OK;
-		if (4.0 * (spk::ss_bands(I.h) + 1) * spk::ss_band_floats(I.w, KT) >= 4.0e9) return SP_OK;
+		if (4.0 * (spk::ss_bands(I.h) + 1) * spk::ss_band_floats(I.w, KT) >= (sum ? 1.0e9 : 4.0e9))
+			return SP_OK;
 	}
 	std::vector<spk::SsBlock> bw;
 	struct Key { int key; spk::SsTask t; };
@@ -685,6 +702,11 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op)
 		spk::launch_ss_clear(ss.op, I.C, (nb + 1) * BS, nullptr);
 		TRY(pl.alloc(&I.bz, (size_t)2 * I.nslot * I.U * KT));
 		const int nT = (T + KT - 1) / KT;
+		if (sum) {
+			I.hs = (nb + 1) * BS;
+			const int last = T - (nT - 1) * KT;   // sweeps of the last block
+			TRY(pl.alloc(&I.hist, ((size_t)(nT - 1) * KT + (last + K - 1) / K * K) * I.hs));
+		}
 		prog_off.push_back(nprog);
 		nprog += (size_t)nT * I.nslot * spk::SS_PS;
 		for (int tb = 0; tb < nT; tb++) {
@@ -728,16 +750,18 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op)
 	for (const spk::SsInst &I : in)
 		if (op != spk::SS_AMLE && !(I.t <= 0.25f)) ss.small = false;
 	ss.nbw = (int)bw.size();
-	ss.blocks = spk::ss_blocks(ss.form, ss.op);
+	ss.blocks = spk::ss_blocks(ss.form, ss.op, sum);
 	ss.nt = (int)tl.size();
 	return SP_OK;
 }
 
-static void ss_run(Plan &pl, const SsRun &ss, const spk::SsInst *d_inst, hipStream_t s)
+static void ss_run(Plan &pl, const SsRun &ss, const spk::SsInst *d_inst, hipStream_t s,
+		int nsum = 0)
 {
 	spk::launch_ss_in(ss.op, d_inst, ss.d_bw, ss.nbw, s);
-	spk::launch_ss_run(ss.form, ss.op, ss.small, ss.d_tasks, ss.nt, ss.blocks, d_inst,
+	spk::launch_ss_run(ss.form, ss.op, ss.sum, ss.small, ss.d_tasks, ss.nt, ss.blocks, d_inst,
 			ss.d_claim, ss.d_mx, GS_FLOW_SPIN, pl.gs_err, s);
+	if (ss.sum) spk::launch_ss_sum(d_inst, ss.d_bw, ss.nbw, nsum, s);
 	spk::launch_ss_out(d_inst, ss.d_bw, ss.nbw, (unsigned *)ss.d_prog, ss.nprog + 3, s);
 }
 
@@ -751,9 +775,10 @@ static int ss_level(Plan &pl, LevelPlan &L, bool has_f)
 		spk::SsInst I{};
 		I.u = L.sp[m].u; I.c = L.sp[m].c;
 		I.w = L.sp[m].w; I.h = L.sp[m].h; I.T = L.nsweep[m]; I.t = pl.teff;
+		if (!pl.acc.empty()) I.acc = pl.acc[L.members[m]];
 		in.push_back(I);
 	}
-	return ss_build(pl, L.ss, in, has_f ? spk::SS_POISSON : spk::SS_LAPLACE);
+	return ss_build(pl, L.ss, in, has_f ? spk::SS_POISSON : spk::SS_LAPLACE, !pl.acc.empty());
 }
 
 // ---------------------------------------------------------- autotuner
@@ -1047,20 +1072,33 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 		std::vector<GsInst> gi(nm);
 		for (int m = 0; m < nm; m++)
 			gi[m] = {L.sp[m].u, L.sp[m].c, L.sp[m].w, L.sp[m].h, L.nsweep[m],
-				pl.teff, nullptr};
+				pl.teff, nullptr, pl.acc.empty() ? nullptr : pl.acc[L.members[m]]};
 		TRY(pl.upload(&L.d_insts, gi));
 		L.insts = gi;
 		// Gauss-Seidel: members that fit in LDS run whole; others in tiles.
 		// For R = 1 the whole-level kernel deals the unknown pixels to the
 		// threads (k_gs_cells), for levels of up to GSC_MAXCELLS pixels
-		std::vector<int> small;
-		const bool cells = pl.R == 1 && g_gsc_lds > 0;
+		std::vector<int> small, diag;
+		const bool cells = pl.R == 1 && g_gsc_lds > 0, sum = !pl.acc.empty();
 		if (cells) {
 			int th = 64, maxs = 1, lds = 0;
 			for (int m = 0; m < nm; m++) {
 				const int w = L.sp[m].w, h = L.sp[m].h, T = L.nsweep[m];
 				if (T <= 0) continue;
-				if ((long)w * h <= GSC_MAXCELLS && gsc_lds_bytes(w, h) <= g_gsc_lds
+				// few sweeps against the level's diagonals: by diagonal (the
+				// form that sums has no other)
+				const int dl = g_gsd_lds > 0 ? spk::gs_diag_lds(w, h, T, has_f, sum) : 0;
+				if (dl > 0 && dl <= g_gsd_lds && (sum || 4 * T <= w + h)) {
+					diag.push_back(m);
+					L.diag_lds = std::max(L.diag_lds, dl);
+					// a step updates the holes among T min(w, h) pixels, and a
+					// thread takes 16 pixels at most
+					const long a = std::min(1024L, std::max((long)T * std::min(w, h) / 2,
+							((long)w * h + 15) / 16));
+					L.diag_threads = std::max(L.diag_threads, (int)((a + 63) / 64 * 64));
+					continue;
+				}
+				if (!sum && (long)w * h <= GSC_MAXCELLS && gsc_lds_bytes(w, h) <= g_gsc_lds
 						&& small_nsteps(1, w, h, T) < 0x7fffffffL) {
 					small.push_back(m);
 					th = std::max(th, gsc_threads(w, h));
@@ -1080,7 +1118,7 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 			// whole level in one work-group: it fits in LDS, every thread
 			// holds at most SMALL_MAXSLOT slots, and the step count fits int
 			const long slots = (long)h * ((w - 1) / (pl.R * pl.R + 1) + 1);
-			if ((long)8 * small_cells(pl.R, w, h) <= g_max_lds
+			if (!sum && (long)8 * small_cells(pl.R, w, h) <= g_max_lds
 					&& slots <= 1024L * SMALL_MAXSLOT
 					&& small_nsteps(pl.R, w, h, T) < 0x7fffffffL) {
 				small.push_back(m);
@@ -1092,6 +1130,9 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 			}
 			L.tiled.push_back(m);
 		}
+		L.ndiag = (int)diag.size();
+		L.diag_fdat = has_f;
+		TRY(pl.upload(&L.d_diag, diag));
 		L.nsmall = (int)small.size();
 		TRY(pl.upload(&L.d_small, small));
 		TRY(ss_level(pl, L, has_f));
@@ -1125,9 +1166,13 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 	return SP_OK;
 }
 
-static int run_gs(Plan &pl, LevelPlan &L, hipStream_t s)
+// nsum (plans with acc): the first sweeps whose values are added up
+static int run_gs(Plan &pl, LevelPlan &L, hipStream_t s, int nsum = 0)
 {
 	if (pl.P.autotune && !L.gs_tuned && L.wf_off.size() > 1) TRY(gs_tune(pl, L, s));
+	if (L.ndiag)
+		spk::launch_gs_diag(L.diag_fdat, !pl.acc.empty(), L.d_insts, L.d_diag, L.ndiag,
+				L.diag_lds, L.diag_threads, nsum, s);
 	if (L.nsmall && L.cells_slots)
 		spk::launch_gs_cells(L.cells_slots, L.d_insts, L.d_small, L.nsmall, L.small_lds,
 				L.small_threads, s);
@@ -1137,7 +1182,7 @@ static int run_gs(Plan &pl, LevelPlan &L, hipStream_t s)
 	if (L.ss.nt) {
 		// algorithmic bytes: as for the tiles, per block of sweeps
 		ProfScope pr("gs_tile", s);
-		ss_run(pl, L.ss, L.ss.d_inst, s);
+		ss_run(pl, L.ss, L.ss.d_inst, s, nsum);
 		pl.gs_flow_used = true;
 		double px = 0;
 		int K, KT;
@@ -2060,13 +2105,20 @@ struct AsLevel {
 	float *v = nullptr, *gg = nullptr, *gf = nullptr, *gi = nullptr;
 	float *g_rot = nullptr, *f_rot = nullptr, *u_rot = nullptr, *acc = nullptr;
 	Plan *sweep = nullptr;      // one sweep of the turned planes, this size
+	// the sweeps without data that follow, `group` of them at once and the
+	// rest of them, their values added to acc (null: swept one by one)
+	Plan *sum = nullptr, *rest = nullptr;
+	int group = 0;
 };
 
 struct AsScratch {
 	std::vector<int> key;       // w, h, pd, levels, niter, PONLIT
 	Plan mem;                   // owns the level buffers
 	std::vector<AsLevel> lv;
-	~AsScratch() { for (auto &L : lv) delete L.sweep; }
+	~AsScratch()
+	{
+		for (auto &L : lv) { delete L.sweep; delete L.sum; delete L.rest; }
+	}
 };
 static std::mutex g_as_mu;
 static AsScratch *g_as = nullptr;
@@ -2117,6 +2169,27 @@ static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 				L.u_rot + L.n * l});
 		L.sweep = new Plan;
 		rc = plan_create(*L.sweep, planes, P1, true);
+		if (rc) break;
+		// the summing sweeps hold the values after each of them: at most
+		// 1 GiB per call
+		L.group = (int)std::min<double>(L.nsweep, std::max(1.0, 2.4e8 / (1.2 * m)));
+		for (PlaneIn &q : planes) q.f = nullptr;
+		for (int part = 0; part < 2 && !rc; part++) {
+			sp_params P2 = P1;
+			P2.niter = part ? L.nsweep % L.group : L.group;
+			if (!P2.niter) break;
+			Plan *pl = new Plan;
+			(part ? L.rest : L.sum) = pl;
+			for (int l = 0; l < pd; l++) pl->acc.push_back(L.acc + L.n * l);
+			rc = plan_create(*pl, planes, P2, false);
+			// planes that the summing forms do not take
+			if (!rc && !pl->lv[0].tiled.empty() && !pl->lv[0].ss.nt) {
+				delete L.sum;
+				delete L.rest;
+				L.sum = L.rest = nullptr;
+				break;
+			}
+		}
 	}
 	if (rc) { delete A; return rc; }
 	g_as = A;
@@ -2159,6 +2232,22 @@ static int adjoint_sweeps_image(const sp_adjoint_image &I, const sp_params &P,
 			spk::as_setup(L.hole, L.v, L.gg, L.g_rot, L.f_rot, L.w, L.h, np, s);
 			TRY(as_sweep(L, true, true, s));            // nu_n = (I/t + U)^-1 lambda
 			spk::as_acc(L.acc, L.u_rot, L.n, np, 1, s);
+			if (L.sum) {   // data 0 from here on
+				for (int done = 0; done < L.nsweep;) {
+					Plan &pl = L.nsweep - done >= L.group ? *L.sum : *L.rest;
+					LevelPlan &L0 = pl.lv[0];
+					spk::launch_prepare(L0.d_sp, L0.d_bw, L0.nbw, L0.d_bcnt, s);
+					const int T = L0.nsweep[0];
+					done += T;
+					// (the last sweep's values are nu_0, which is not summed)
+					TRY(run_gs(pl, L0, s, done < L.nsweep ? T : T - 1));
+				}
+				spk::as_finish(L.hole, L.u_rot, L.acc, L.w, L.h, np, t, L.gi, L.gf, L.gg, s);
+				if (k + 1 < nl)
+					spk::as_zoom_in_t(L.gi, L.hole, L.w, L.h, A->lv[k + 1].v, A->lv[k + 1].w,
+							A->lv[k + 1].h, np, s);
+				continue;
+			}
 			spk::as_fill(L.f_rot, L.n, np, 0.0f, s);    // data 0 from here on
 			for (int j = 1; j < L.nsweep; j++) {
 				TRY(as_sweep(L, j == 1, false, s));

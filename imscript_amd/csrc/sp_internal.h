@@ -268,6 +268,14 @@ int small_lds_bytes(int R, int w, int h);
 int gs_cells_enable(int bytes);
 void launch_gs_cells(int maxs, const GsInst *insts, const int *ids, int nids,
 		int lds_bytes, int threads, hipStream_t s);
+// whole R = 1 levels by diagonal (k_gs_diag): LDS bytes, allow them (0 on
+// success), launch.  fdat: with data terms; sum (without data terms): adds
+// the values of the first nsum sweeps to each plane's acc
+// (0: the level is beyond them)
+int gs_diag_lds(int w, int h, int T, bool fdat, bool sum);
+int gs_diag_enable(int bytes);
+void launch_gs_diag(bool fdat, bool sum, const GsInst *insts, const int *ids, int nids,
+		int lds_bytes, int threads, int nsum, hipStream_t s);
 void launch_gs_tiles(int R, int var, const GsTile *tiles, int ntiles,
 		const GsInst *insts, hipStream_t s);
 void launch_gs_small(int R, const GsInst *insts, const int *ids, int nids,

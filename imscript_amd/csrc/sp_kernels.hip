@@ -540,6 +540,150 @@ __global__ __launch_bounds__(GSC_MAXNT) void k_gs_cells(const GsInst *insts, con
 	gsc_store<MAXS>(th, in);
 }
 
+// Whole R = 1 level by diagonal, for few sweeps.  k_gs_cells walks all of a
+// thread's pixels on every step, of which few are under way when the sweeps
+// are few against the level's i + j.  Here the unknowns are listed by i + j
+// (even sums first), so the pixels of step s, whose sums lie in
+// [s - 2 (T - 1), s] with the parity of s, are one stretch of the list, and a
+// step is one or two of its entries per thread: the level's values stay in LDS
+// (96 x 128, 10 sweeps: 67 us, by k_gs_cells 111; 128 x 128: 40 sweeps 168 and
+// 246, 60 sweeps 204 and 282 for the whole call).  Bound: the instructions of a
+// step, most of whose wavefronts have none or one entry each.  FDAT: data term
+// from LDS.  SUM: a pixel's values after sweeps 0..nsum-1 are added to acc one
+// by one.
+constexpr int GSD_MAXDIAG = 1024;    // W + H at most
+constexpr int GSD_PX = 16;           // pixels per thread at most
+constexpr int GSD_MAXSTEPS = 3072;   // W + H + 2 T at most
+
+template <bool FDAT, bool SUM>
+__global__ __launch_bounds__(GSC_MAXNT) void k_gs_diag(const GsInst *insts, const int *ids,
+		int nsum)
+{
+	extern __shared__ float smem[];
+	__shared__ int off[GSD_MAXDIAG + 2], wsum[16];
+	__shared__ unsigned tab[GSD_MAXSTEPS + 2];
+	const GsInst in = insts[ids[blockIdx.x]];
+	const int W = in.w, H = in.h, T = in.nsweep, P = W + 2, n = W * H;
+	if (T <= 0) return;
+	const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
+	const int nf = P * (H + 2);   // values, data terms and sums in a frame
+	float *U = smem, *C = U + nf, *A = C + (FDAT ? nf : 0);
+	unsigned *L = (unsigned *)(A + (SUM ? nf : 0));
+	const int D = W + H - 1, De = (D + 1) >> 1;   // diagonals, even ones
+	// the thread's pixels tid, tid + nt, ...: their loads go out together
+	float uv[GSD_PX], cv[GSD_PX];
+#pragma unroll
+	for (int m = 0; m < GSD_PX; m++) {
+		const int q = min(tid + m * nt, n - 1);
+		uv[m] = gload<float>(in.u + q);
+		cv[m] = gload<float>(in.c + q);
+	}
+	for (int d = tid; d <= D; d += nt) off[d] = 0;
+	for (int x = tid; x < P; x += nt) U[x] = U[(H + 1) * P + x] = sp_float(SP_QNAN_BITS);
+	for (int y = tid; y < H; y += nt)
+		U[(y + 1) * P] = U[(y + 1) * P + W + 1] = sp_float(SP_QNAN_BITS);
+	__syncthreads();
+	// place of diagonal d in the list's order
+	auto place = [&](int d) { return d & 1 ? De + (d >> 1) : d >> 1; };
+	unsigned ent[GSD_PX];   // framed index | (i + j) << 16; 0: known, or none
+#pragma unroll
+	for (int m = 0; m < GSD_PX; m++) {
+		const int q = tid + m * nt;
+		ent[m] = 0;
+		if (q >= n) continue;
+		const int j = q / W, i = q - j * W, p = (j + 1) * P + i + 1;
+		U[p] = uv[m];
+		if (FDAT) C[p] = cv[m];
+		if (SUM) A[p] = in.acc[q];
+		if (sp_known(cv[m])) continue;
+		ent[m] = (unsigned)p | (unsigned)(i + j) << 16;
+		atomicAdd(&off[place(i + j)], 1);
+	}
+	__syncthreads();
+	// counts to starts, in chunks of the work-group
+	for (int base = 0, run = 0; base <= D; base += nt) {
+		const int k = base + tid, v = k <= D ? off[k] : 0;
+		int tot;
+		const int pre = block_exscan(v, wsum, &tot);
+		if (k <= D) off[k] = run + pre;
+		run += tot;
+		__syncthreads();
+	}
+	// filling moves a start to its end
+#pragma unroll
+	for (int m = 0; m < GSD_PX; m++)
+		if (ent[m]) L[atomicAdd(&off[place((int)(ent[m] >> 16))], 1)] = ent[m];
+	__syncthreads();
+	// now off[k] is the end of place k, and the start of place k + 1
+	const int ns = (int)small_nsteps(1, W, H, T);
+	// the stretch [x, y) of each step, as x | y << 16
+	for (int s = tid; s < ns + 2; s += nt) {
+		int lo = s - 2 * (T - 1), hi = min(s, D - 1);
+		lo = lo < 0 ? s & 1 : lo;
+		hi -= (hi ^ s) & 1;
+		const int k = place(lo);
+		tab[s] = lo > hi || s >= ns ? 0u : (unsigned)(k ? off[k - 1] : 0)
+			| (unsigned)off[place(hi)] << 16;
+	}
+	__syncthreads();
+	// a wavefront's entries of a step; those of the next step and the stretch
+	// of the one after are read along with this step's values
+	const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63);
+	unsigned r = __builtin_amdgcn_readfirstlane((int)tab[0]);
+	unsigned r1 = __builtin_amdgcn_readfirstlane((int)tab[1]);
+	unsigned q = L[min((int)(r & 0xffffu) + tid, n - 1)];
+	for (int s = 0; s < ns; s++) {
+		const unsigned qn = L[min((int)(r1 & 0xffffu) + tid, n - 1)], r2 = tab[s + 2];
+		const int b = (int)(r >> 16);
+		for (int e0 = (int)(r & 0xffffu) + wave0; e0 < b; e0 += nt) {
+			const int e = e0 + (tid & 63);
+			if (e0 != (int)(r & 0xffffu) + wave0) q = L[min(e, n - 1)];
+			if (e < b) {
+				const int p = (int)(q & 0xffffu);
+				const float y = gsc_update(U, p, P, U[p], FDAT ? C[p] : 0.0f, in.t);
+				U[p] = y;
+				if (SUM && (s - (int)(q >> 16)) >> 1 < nsum) A[p] = A[p] + y;
+			}
+		}
+		__syncthreads();
+		r = r1;
+		r1 = __builtin_amdgcn_readfirstlane((int)r2);
+		q = qn;
+	}
+#pragma unroll
+	for (int m = 0; m < GSD_PX; m++) {
+		if (!ent[m]) continue;
+		const int q = tid + m * nt, p = (int)(ent[m] & 0xffffu);
+		in.u[q] = U[p];
+		if (SUM) in.acc[q] = A[p];
+	}
+}
+
+int gs_diag_lds(int w, int h, int T, bool fdat, bool sum)
+{
+	if ((long)w * h > GSC_MAXCELLS || w + h > GSD_MAXDIAG || w + h + 2L * T > GSD_MAXSTEPS)
+		return 0;
+	return 4 * ((w + 2) * (h + 2) * (1 + fdat + sum) + w * h);
+}
+
+int gs_diag_enable(int bytes)
+{
+	for (const void *f : {(const void *)k_gs_diag<false, false>,
+			(const void *)k_gs_diag<true, false>, (const void *)k_gs_diag<false, true>})
+		if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes)
+				!= hipSuccess)
+			return -1;
+	return 0;
+}
+
+void launch_gs_diag(bool fdat, bool sum, const GsInst *insts, const int *ids, int nids,
+		int lds_bytes, int threads, int nsum, hipStream_t s)
+{
+	if (sum) k_gs_diag<false, true><<<nids, threads, lds_bytes, s>>>(insts, ids, nsum);
+	else if (fdat) k_gs_diag<true, false><<<nids, threads, lds_bytes, s>>>(insts, ids, 0);
+	else k_gs_diag<false, false><<<nids, threads, lds_bytes, s>>>(insts, ids, 0);
+}
+
 // slots per thread and parity of the compiled instances
 static int gsc_inst(int maxs) { return maxs <= 1 ? 1 : maxs <= 2 ? 2 : maxs <= 4 ? 4 : 8; }
 

@@ -52,6 +52,9 @@ struct SsInst {
 	unsigned BS;         // floats per band
 	int pad;             // steps of padding before i = 0
 	int U, nslot;        // bz: steps per band, bands per block of sweeps
+	float *hist;         // the values after every sweep, hs floats each, or null
+	size_t hs;
+	float *acc;          // image layout: where they are added up
 };
 struct SsTask { int inst, tb, J; };   // band J of the tb-th block of sweeps
 struct SsBlock { int inst, jb, sb; }; // 64 x 64 block of the skewed layout
@@ -64,14 +67,17 @@ inline int ss_steps(int w, int KT) { return w + KT + 2 * 64 + 5 * SS_C; }
 inline int ss_bands(int h) { return (h + 63) / 64; }
 inline size_t ss_band_floats(int w, int KT) { return (size_t)64 * (w + 63 + 2 * ss_pad(KT)); }
 
-int ss_blocks(int form, int op);   // work-groups that can be resident
+int ss_blocks(int form, int op, bool sum);   // work-groups that can be resident
 void launch_ss_clear(int op, float *C, size_t n, hipStream_t s);
 void launch_ss_in(int op, const SsInst *in, const SsBlock *bw, int nb, hipStream_t s);
 // small: the step and the sweeps are such that values bounded by those the
 // kernels test for stay small; mx: the level's largest |value| and |data term|
-void launch_ss_run(int form, int op, bool small, const SsTask *tasks, int nt, int blocks,
+// sum (SS_LAPLACE): also writes hist
+void launch_ss_run(int form, int op, bool sum, bool small, const SsTask *tasks, int nt, int blocks,
 		const SsInst *in, unsigned *claim, const unsigned *mx, int spin_max, int *err,
 		hipStream_t s);
+// acc += the values after sweeps 0..nsum-1, one by one, at the swept pixels
+void launch_ss_sum(const SsInst *in, const SsBlock *bw, int nb, int nsum, hipStream_t s);
 // also sets words[0, nwords) (the progress words, claim and mx) to 0
 void launch_ss_out(const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
 		int nwords, hipStream_t s);

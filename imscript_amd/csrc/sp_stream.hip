@@ -203,10 +203,11 @@ struct SsLds {
 
 // SS_C steps from the coefficient row crow on.  cv: the coefficients of the next SS_C
 // steps, each replaced after its use by the one SS_C steps on (crow + its offset).
-template <int K, int OP, int FORM>
+template <int K, int OP, int FORM, bool SUM>
 static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_C][K],
 		__amdgpu_buffer_rsrc_t cbuf, unsigned crow, const unsigned (&voff)[K], const SsLds &l,
-		int lane, float t, int i0, int jrow, int W, int H)
+		int lane, float t, int i0, int jrow, int W, int H, __amdgpu_buffer_rsrc_t hbuf,
+		unsigned hs4)
 {
 	constexpr int KP = K <= 4 ? 4 : 8;
 	float zi[K], zm, ym;
@@ -238,6 +239,9 @@ static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_C]
 #pragma unroll
 		for (int k = 0; k < K; k++) {
 			cv[c][k] = ss_coef(cbuf, voff[k], crow + (c + SS_C) * 256);
+			if (SUM)
+				__builtin_amdgcn_raw_buffer_store_b32(__float_as_int(yn[k]), hbuf, voff[k],
+						crow + c * 256 + k * hs4, 0);
 			q.Y[k] = yn[k];
 			q.Z[k] = zn[k];
 		}
@@ -258,7 +262,7 @@ static __device__ __forceinline__ void ss_chunk(SsState<K> &q, float (&cv)[SS_C]
 	}
 }
 
-template <int K, int NW, int OP>
+template <int K, int NW, int OP, bool SUM>
 __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_ss_run(const SsTask *tasks, int nt,
 		const SsInst *insts, unsigned *claim, const unsigned *mx, int spin_max, int *err)
 {
@@ -328,6 +332,10 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 				__builtin_amdgcn_s_waitcnt(0);
 			}
 			ss_barrier();
+			const unsigned hs4 = SUM ? 4u * (unsigned)(nb + 1) * BS : 0u;
+			const __amdgpu_buffer_rsrc_t hbuf = __builtin_amdgcn_make_buffer_rsrc(
+					SUM ? ss_uni(ip->hist) + (size_t)kw * (hs4 / 4) : pC, 0, (int)(K * hs4),
+					0x00027000);
 			auto run = [&](auto form, int pa, int pb) {
 				for (int p = pa; p < pb; p++) {
 					if (wv < nwa && p >= wv && p - wv < nch) {
@@ -335,9 +343,9 @@ __global__ __launch_bounds__((NW + 2) * 64) __attribute__((amdgpu_waves_per_eu(4
 							&zin[wv][(wv ? p - 1 : p) & 3][0][0],
 							&line[wv + 1][(p + 1) & 1][0][0], &zo[wv][(p + 1) & 1][0][0]};
 						const int s0 = (gs + p - wv) * C;
-						ss_chunk<K, OP, decltype(form)::value>(st, cv, cbuf,
+						ss_chunk<K, OP, decltype(form)::value, SUM>(st, cv, cbuf,
 								cbase + 256u * (unsigned)s0, voff, l, lane, t,
-								s0 - jrow - 2 * kw, jrow, W, H);
+								s0 - jrow - 2 * kw, jrow, W, H, hbuf, hs4);
 					}
 					ss_barrier();
 				}
@@ -564,6 +572,43 @@ __global__ __launch_bounds__(256) void k_ss_in(const SsInst *insts, const SsBloc
 	}
 }
 
+// acc += the values after each of the first nsum sweeps at the swept pixels,
+// in that order
+__global__ __launch_bounds__(256) void k_ss_sum(const SsInst *insts, const SsBlock *bw, int nsum)
+{
+	__shared__ float sa[64][65];
+	const SsBlock b = bw[blockIdx.x];
+	const SsInst in = insts[b.inst];
+	const int lane = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+	float a[16];
+#pragma unroll
+	for (int r = 0; r < 16; r++) {
+		const int jr = r0 + 4 * r, j = b.jb * 64 + jr, i = b.sb * 64 + lane - jr;
+		a[r] = gload<float>(in.acc + (size_t)sp_clamp(j, 0, in.h - 1) * in.w
+				+ sp_clamp(i, 0, in.w - 1));
+	}
+#pragma unroll
+	for (int r = 0; r < 16; r++) sa[r0 + 4 * r][lane] = a[r];
+	__syncthreads();
+	const float *h = in.hist + (size_t)b.jb * in.BS + (size_t)(b.sb * 64 + in.pad + r0) * 64 + lane;
+#pragma unroll
+	for (int r = 0; r < 16; r++) a[r] = sa[lane][r0 + 4 * r];
+	for (int k = 0; k < nsum; k++, h += in.hs)
+#pragma unroll
+		for (int r = 0; r < 16; r++) a[r] = a[r] + gload<float>(h + r * 256);
+	__syncthreads();
+#pragma unroll
+	for (int r = 0; r < 16; r++) sa[lane][r0 + 4 * r] = a[r];
+	__syncthreads();
+#pragma unroll
+	for (int r = 0; r < 16; r++) {
+		const int jr = r0 + 4 * r, j = b.jb * 64 + jr, i = b.sb * 64 + lane - jr;
+		if (j >= in.h || i < 0 || i >= in.w) continue;
+		const size_t p = (size_t)j * in.w + i;
+		if (!sp_known(in.c[p])) in.acc[p] = sa[jr][lane];
+	}
+}
+
 // the swept pixels back to the image layout
 // (and the words of the next run's synchronisation back to 0)
 __global__ __launch_bounds__(256) void k_ss_out(const SsInst *insts, const SsBlock *bw,
@@ -596,17 +641,18 @@ __global__ __launch_bounds__(256) void k_ss_out(const SsInst *insts, const SsBlo
 	}
 }
 
-template <class F> static void ss_with(int form, int op, F &&f)
+template <class F> static void ss_with(int form, int op, bool sum, F &&f)
 {
 	sp_with_form(form, [&](auto fm) {
 		constexpr int K = decltype(fm)::K, NW = decltype(fm)::NW;
-		if (op == SS_LAPLACE) f(k_ss_run<K, NW, SS_LAPLACE>, (NW + 2) * 64);
-		else if (op == SS_AMLE) f(k_ss_run<K, NW, SS_AMLE>, (NW + 2) * 64);
-		else f(k_ss_run<K, NW, SS_POISSON>, (NW + 2) * 64);
+		if (sum) f(k_ss_run<K, NW, SS_LAPLACE, true>, (NW + 2) * 64);
+		else if (op == SS_LAPLACE) f(k_ss_run<K, NW, SS_LAPLACE, false>, (NW + 2) * 64);
+		else if (op == SS_AMLE) f(k_ss_run<K, NW, SS_AMLE, false>, (NW + 2) * 64);
+		else f(k_ss_run<K, NW, SS_POISSON, false>, (NW + 2) * 64);
 	});
 }
 
-int ss_blocks(int form, int op)
+int ss_blocks(int form, int op, bool sum)
 {
 	int nb = INT_MAX;
 	auto ask = [&](auto *k, int threads) {
@@ -619,7 +665,7 @@ int ss_blocks(int form, int op)
 			ncu = 256;
 		nb = std::min(nb, std::max(1, per) * ncu);
 	};
-	ss_with(form, op, ask);
+	ss_with(form, op, sum, ask);
 	return nb;
 }
 
@@ -634,7 +680,7 @@ void launch_ss_in(int op, const SsInst *in, const SsBlock *bw, int nb, hipStream
 	else k_ss_in<SS_POISSON><<<nb, 256, 0, s>>>(in, bw);
 }
 
-void launch_ss_run(int form, int op, bool small, const SsTask *tasks, int nt, int blocks,
+void launch_ss_run(int form, int op, bool sum, bool small, const SsTask *tasks, int nt, int blocks,
 		const SsInst *in, unsigned *claim, const unsigned *mx, int spin_max, int *err,
 		hipStream_t s)
 {
@@ -642,7 +688,12 @@ void launch_ss_run(int form, int op, bool small, const SsTask *tasks, int nt, in
 		k<<<std::min(nt, blocks), threads, 0, s>>>(tasks, nt, in, claim, small ? mx : nullptr,
 				spin_max, err);
 	};
-	ss_with(form, op, run);
+	ss_with(form, op, sum, run);
+}
+
+void launch_ss_sum(const SsInst *in, const SsBlock *bw, int nb, int nsum, hipStream_t s)
+{
+	if (nsum > 0) k_ss_sum<<<nb, 256, 0, s>>>(in, bw, nsum);
 }
 
 void launch_ss_out(const SsInst *in, const SsBlock *bw, int nb, unsigned *words,
