@@ -61,6 +61,8 @@ constexpr int MG_FINE_TX[MG_NFINE] = {120, 120, 116, 112, 108, 104};
 constexpr int MG_FINE_TY[MG_NFINE] = {56, 56, 52, 48, 44, 40};
 constexpr int MG_FINE_NU[MG_NFINE] = {2, 2, 3, 4, 5, 6};
 constexpr int MG_FINE_T[MG_NFINE] = {512, 1024, 1024, 1024, 1024, 1024};
+// the fine shape that level 0 may also run by one wave per tile
+constexpr int MG_STRIP_GEO = 4;
 constexpr int MG_NGEO = 6;
 constexpr int MG_GEO_TX[MG_NGEO] = {112, 112, 112, 48, 104, 40};
 constexpr int MG_GEO_TY[MG_NGEO] = {32, 32, 48, 16, 40, 8};
@@ -136,6 +138,8 @@ struct Cg32Batch {
 	int4 *tiles0;      // level-0 tiles (plane, x0, y0, -), contiguous per plane
 	int ntiles0;
 	int geo0;          // their shape (MG_FINE_*)
+	int strips0;       // one wave per tile (shape MG_STRIP_GEO only)
+	int odd0;          // some plane has an odd width
 	double *tpart;     // one partial per level-0 tile
 	double px0;        // level-0 pixels of the batch (profiler bytes)
 	ProfFn prof;

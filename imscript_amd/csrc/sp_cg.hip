@@ -335,12 +335,14 @@ __global__ __launch_bounds__(NT) void k32_setup(const BlockWork *bw,
 		// right-hand side), x only in groups with an unknown.  The
 		// biharmonic iteration starts from p = r, and its product reads p
 		// at every pixel of the 13-point stencil, unknown or not: p and q
-		// everywhere.  (The Poisson iteration writes p and q itself.)
+		// everywhere, and z, of which p takes whole groups.  (The Poisson
+		// iteration writes p and q itself.)
 		gstore<unsigned>(P.code + q4, cc);
 		gstore<f4>(P.r + q4, rv);
 		if (P.bilap) {
 			gstore<f4>(P.p + q4, rv);
 			gstore<f4>(P.q + q4, f4{0.0f, 0.0f, 0.0f, 0.0f});
+			if (P.z != P.r) gstore<f4>(P.z + q4, f4{0.0f, 0.0f, 0.0f, 0.0f});
 		}
 		if (cc & 0x01010101u) gstore<d4>(P.x + q4, xv);
 	}
@@ -1650,7 +1652,6 @@ void k_mg_down(const int4 *tiles,
 		if (I < Cc.w && J < Cc.h) {
 			const size_t cq = (size_t)J * Cc.w + I;
 			gstore<float>(Cc.b + cq, acc);
-			gstore<float>(Cc.z + cq, 0.0f);
 		}
 	}
 }
@@ -1666,7 +1667,7 @@ void k_mg_up(const int4 *tiles, const MgLevel *lv,
 		const MgLevel *coarse, const Cg32Scal *sc, float wc, double *tpart)
 {
 	__shared__ float z[G::ZN];
-	__shared__ double red[G::T / 64];
+	__shared__ double red[DOT ? G::T / 64 : 1];
 	const int tb = xcd_block();
 	const int4 t = tiles[tb];
 	const MgLevel L = lv[t.x], Cc = coarse[t.x];
@@ -1705,9 +1706,329 @@ void k_mg_up(const int4 *tiles, const MgLevel *lv,
 				acc += (double)C.b[kb][c] * z[cell_z(C, kb, c)];
 		}
 	}
-	if (DOT) {
+	if constexpr (DOT && G::K == 2 && G::PAIRS_X == 64) {
+		// four rows a thread: the groups of four rows of a column pair
+		// downwards, then the 64 pairs (the order that one wave takes in
+		// k_mg0_strip)
+		__shared__ double grp[G::T];
+		grp[threadIdx.x] = acc;
+		__syncthreads();
+		if (threadIdx.x < 64) {
+			double v = 0;
+			for (int m = 0; m < G::RG; m++) v += grp[m * 64 + threadIdx.x];
+			for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+			if (threadIdx.x == 0) tpart[tb] = v;
+		}
+	} else if constexpr (DOT) {
 		const double sum = bsum<G::T>(acc, red);
 		if (threadIdx.x == 0) tpart[tb] = sum;
+	}
+}
+
+// ------------------------------------------- level 0 by streaming strips
+//
+// The level-0 smoother (nu = 5) of a tile of 108 x 44 by one wave, without
+// barriers.  Lane c holds columns 2c and 2c + 1 of the 128 (the tile and its
+// halo of 10 on each side) and the wave runs down the rows once.  Every half
+// sweep follows the one before it by a row: in step t the pre-smoother's half
+// sweep h runs on row t - h, the post-smoother's on row t - 1 - h, so the rows
+// above have had it and the rows below have had half sweep h - 1, as in whole
+// half sweeps, and one step updates the same column of the pair in all ten
+// rows.  z, b and 1/diagonal of the rows in flight are registers (rings of
+// M0_U rows; the steps are unrolled M0_U times, so every ring index is a
+// constant); the vertical neighbours are the lane's own registers, the
+// horizontal ones its own or the next lane's (one DPP operand): five
+// operations an update, against about nine, 1.5 LDS reads and a barrier per
+// half sweep in the tile kernels.  The sums are those of mg_half in its
+// order, so z keeps the bits of the tile kernels.
+//
+// A pair of known pixels (code 0) has its b and z neither read nor written
+// (an offset beyond the buffer: such a load returns 0, such a store is
+// dropped), so z and zd hold values at pairs with an unknown only.
+//
+// 3 x 4096 x 4096, half of it unknown, a launch: down 106 us, up 127 us; by
+// the tile kernels 176 and 198.  With neither loads nor stores the launches
+// take 77 and 71 us (the operations: 2.5 cycles for a plain one, 4.4 for a
+// DPP one), without the stores alone 79 and 98: what is left over them is
+// the stores, 155 MB in short rows.  The depth of the loads (2 to 8 rows), the
+// height of a strip (44 to 132 rows: less halo, fewer waves) and leaving out
+// rows without an unknown in flight measured the same or slower.
+constexpr int M0_NU = 5, M0_HALO = 2 * M0_NU, M0_TX = 128 - 2 * M0_HALO, M0_U = 24;
+constexpr int M0_TY = MG_FINE_TY[MG_STRIP_GEO];
+constexpr int M0_BA = 4, M0_CA = 7;      // rows that b / codes are ahead
+constexpr unsigned M0_OFF = 0xfffffff0u; // beyond every buffer
+static_assert(M0_CA + 2 * M0_NU + 1 < M0_U, "ring too short");
+static_assert(M0_TX == MG_FINE_TX[MG_STRIP_GEO] && M0_NU == MG_FINE_NU[MG_STRIP_GEO]
+		&& M0_TY % 4 == 0, "strips are the default tiles");
+
+constexpr int m0_at(int k) { return (k + 2 * M0_U) % M0_U; }
+
+static __device__ __forceinline__ float m0_west(float v)   // lane - 1
+{
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+
+static __device__ __forceinline__ float m0_east(float v)   // lane + 1
+{
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+
+// A buffer's descriptor.  Addresses are a lane's byte offset in the row (a
+// register that does not change, or M0_OFF) plus the row's (scalar); a row
+// that is not to be touched has a descriptor of 0 bytes.
+struct M0Buf {
+	uintptr_t p;
+	unsigned n;
+	__device__ __forceinline__ __amdgpu_buffer_rsrc_t row(bool in) const
+	{
+		return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, in ? (int)n : 0, 0x00020000);
+	}
+};
+
+static __device__ __forceinline__ int m0_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+static __device__ __forceinline__ M0Buf m0_buf(const void *p, unsigned bytes)
+{
+	const unsigned long long v = (unsigned long long)(uintptr_t)p;
+	const unsigned lo = (unsigned)m0_uni((int)(unsigned)v), hi = (unsigned)m0_uni((int)(v >> 32));
+	return {(uintptr_t)((unsigned long long)hi << 32 | lo), (unsigned)m0_uni((int)bytes)};
+}
+
+// the rows in flight of one lane's pair, and what its steps need
+template <bool UP, bool EVEN> struct M0Strip {
+	float b0[M0_U], b1[M0_U], z0[M0_U], z1[M0_U], r0[M0_U], r1[M0_U], ce[M0_U / 2];
+	unsigned cd[M0_U], dg[UP ? 1 : M0_U];   // codes; diagonals, a byte each
+	M0Buf code, b, zd, out, cc;
+	const float *lut;                // rdiag of a code byte (LDS)
+	unsigned vc, vb, vo, vl, vk, vko;   // the lane's offsets (see kernel)
+	bool mine, lone;                  // odd width: the pair is the last column alone
+	unsigned sh;                     // its code's shift
+	unsigned w, h, cw, ch;
+	int jt;                          // image row of strip row 0
+	float wc, ca;
+	double acc, tot;                 // r.z of four rows, of the rows before them
+
+	__device__ __forceinline__ bool row_in(int r) const { return (unsigned)(jt + r) < h; }
+	// the row's first pixel; outside the image, where no lane touches any, that
+	// of the nearest row: a scalar offset never exceeds its buffer
+	__device__ __forceinline__ unsigned row_at(int r) const
+	{ return (unsigned)clampi(jt + r, 0, (int)h - 1) * w; }
+	__device__ __forceinline__ unsigned coarse_at(int r) const
+	{ return (unsigned)clampi((jt + r) >> 1, 0, (int)ch - 1) * cw; }
+	template <int K> __device__ __forceinline__ void load_code(int r)
+	{
+		const __amdgpu_buffer_rsrc_t d = code.row(row_in(r));
+		cd[K] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(d, vc, row_at(r), 0);
+	}
+	template <int K> __device__ __forceinline__ void load_row(int r)
+	{
+		if constexpr (!EVEN) cd[K] >>= sh;
+		const unsigned o = cd[K] ? vb : M0_OFF, at = 4u * row_at(r);
+		const gu2 v = __builtin_bit_cast(gu2,
+				__builtin_amdgcn_raw_buffer_load_b64(b.row(true), o, at, 0));
+		b0[K] = __uint_as_float(v.x);
+		b1[K] = __uint_as_float(v.y);
+		if constexpr (UP) {
+			const gu2 y = __builtin_bit_cast(gu2,
+					__builtin_amdgcn_raw_buffer_load_b64(zd.row(true), o, at, 0));
+			z0[K] = __uint_as_float(y.x);
+			z1[K] = __uint_as_float(y.y);
+			if constexpr (!(K & 1))
+				ce[K / 2] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+						cc.row(true), vk, 4u * coarse_at(r), 0));
+		} else {
+			z0[K] = z1[K] = 0.0f;
+		}
+	}
+	template <int K> __device__ __forceinline__ void decode()
+	{
+		r0[K] = lut[cd[K] & 255u];
+		r1[K] = lut[cd[K] >> 8];
+		if constexpr (!UP) dg[K] = (cd[K] >> 5) & 0x0707u;
+	}
+	// half sweep S of step U
+	template <int U, int S> __device__ __forceinline__ void half()
+	{
+		constexpr int k = m0_at(U - S - (UP ? 1 : 0)), no = m0_at(k - 1), so = m0_at(k + 1);
+		if constexpr (!(U & 1)) {
+			float v = b0[k];
+			if constexpr (UP || S > 0) {
+				v += z1[k];
+				v += z0[so];
+				v += m0_west(z1[k]);
+				v += z0[no];
+			}
+			z0[k] = v * r0[k];
+		} else {
+			float v = b1[k];
+			if constexpr (UP || S > 0) {
+				v = m0_east(z0[k]) + v;
+				v += z1[so];
+				v += z0[k];
+				v += z1[no];
+			}
+			z1[k] = v * r1[k];
+		}
+		if constexpr (S + 1 < 2 * M0_NU) this->template half<U, S + 1>();
+	}
+	// step t (t % M0_U == U)
+	template <int U> __device__ __forceinline__ void step(int t)
+	{
+		load_row<m0_at(U + M0_BA)>(t + M0_BA);
+		load_code<m0_at(U + M0_CA)>(t + M0_CA);
+		decode<m0_at(U + 1)>();
+		// row t arrives
+		if constexpr (!EVEN) {
+			b0[U] = lone ? b1[U] : b0[U];
+			b1[U] = lone ? 0.0f : b1[U];
+			if constexpr (UP) {
+				z0[U] = lone ? z1[U] : z0[U];
+				z1[U] = lone ? 0.0f : z1[U];
+			}
+		}
+		if constexpr (UP) {
+			const float e = wc * ce[U / 2];
+			z0[U] += r0[U] != 0.0f ? e : 0.0f;
+			z1[U] += r1[U] != 0.0f ? e : 0.0f;
+		}
+		half<U, 0>();
+		// row t - 2 nu is finished
+		constexpr int k = m0_at(U - 2 * M0_NU), no = m0_at(k - 1), so = m0_at(k + 1);
+		const bool o = t >= 2 * M0_HALO;
+		const __amdgpu_buffer_rsrc_t d = (UP ? out : zd).row(o);
+		const unsigned at = 4u * row_at(t - M0_HALO);
+		const bool any = UP ? r0[k] + r1[k] != 0.0f : dg[UP ? 0 : k] != 0u;
+		__builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(
+				decltype(__builtin_amdgcn_raw_buffer_load_b64(d, 0, 0, 0)),
+				gf2{z0[k], z1[k]}), d, any ? vo : M0_OFF, at, 0);
+		if constexpr (!EVEN)
+			__builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(z0[k]), d,
+					any ? vl : M0_OFF, at, 0);
+		if constexpr (UP) {
+			acc = __builtin_fma((double)b0[k], (double)z0[k], acc);
+			acc = __builtin_fma((double)b1[k], (double)z1[k], acc);
+			if constexpr ((U & 3) == 1) { tot += acc; acc = 0; }
+		} else {
+			float s0 = z1[k] + z0[so], s1 = m0_east(z0[k]) + z1[so];
+			s0 += m0_west(z1[k]);
+			s1 += z0[k];
+			s0 += z0[no];
+			s1 += z1[no];
+			const unsigned g = dg[UP ? 0 : k];
+			// (a known pixel's diagonal is 0, an unknown's at least 2)
+			const float d0 = (float)(g & 255u), d1 = (float)(g >> 8);
+			const float v0 = fminf(d0, 1.0f) * (b0[k] - (d0 * z0[k] - s0));
+			const float v1 = fminf(d1, 1.0f) * (b1[k] - (d1 * z1[k] - s1));
+			ca = U & 1 ? ca + v0 : v0;
+			ca += v1;
+			if constexpr (U & 1) {
+				const bool in = o && (jt + t - M0_HALO) >> 1 < (int)ch;
+				__builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ca), cc.row(in), vko,
+						4u * coarse_at(t - M0_HALO), 0);
+			}
+		}
+	}
+	// four steps; false: the last
+	template <int U> __device__ __forceinline__ bool steps4(int t, int steps)
+	{
+		step<U>(t);
+		__builtin_amdgcn_sched_barrier(0);
+		step<U + 1>(t + 1);
+		__builtin_amdgcn_sched_barrier(0);
+		step<U + 2>(t + 2);
+		__builtin_amdgcn_sched_barrier(0);
+		step<U + 3>(t + 3);
+		__builtin_amdgcn_sched_barrier(0);
+		if constexpr (UP)
+			if (t + 4 <= 2 * M0_HALO) acc = tot = 0;   // rows above the tile
+		return t + 4 < steps;
+	}
+	template <int K> __device__ __forceinline__ void clear()
+	{
+		b0[K] = b1[K] = z0[K] = z1[K] = r0[K] = r1[K] = ce[K / 2] = 0.0f;
+		cd[K] = 0u;
+		if constexpr (!UP) dg[K] = 0u;
+		if constexpr (K + 1 < M0_U) this->template clear<K + 1>();
+	}
+	template <int K> __device__ __forceinline__ void first()
+	{
+		load_code<K>(K);
+		if constexpr (K + 1 < M0_CA) this->template first<K + 1>();
+	}
+	template <int K> __device__ __forceinline__ void first_rows()
+	{
+		load_row<K>(K);
+		if constexpr (K + 1 < M0_BA) this->template first_rows<K + 1>();
+	}
+};
+
+// UP: coarse correction and post-smoothing of zd into z, partial r.z of the
+// tile (in k_mg_up's order: the same bits); else pre-smoothing from 0 into
+// zd, residual, 2 x 2 restriction.  EVEN: every plane has an even width.
+template <bool UP, bool EVEN>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+void k_mg0_strip(const int4 *tiles, const MgLevel *lv, const MgLevel *coarse,
+		const Cg32Scal *sc, float wc, double *tpart)
+{
+	__shared__ float lut[256];
+	const int tb = xcd_block();
+	const int4 tv = tiles[tb];
+	const int4 t4 = make_int4(m0_uni(tv.x), m0_uni(tv.y), m0_uni(tv.z), 0);
+	const MgLevel L = lv[t4.x], C = coarse[t4.x];
+	if (!sc[t4.x].active) return;
+#pragma unroll
+	for (int k = 0; k < 4; k++) lut[threadIdx.x + 64 * k] = Lev0::rdiag(threadIdx.x + 64 * k);
+	const int i0 = t4.y - M0_HALO + 2 * (int)threadIdx.x;
+	const int w = m0_uni(L.w), h = m0_uni(L.h), cw = m0_uni(C.w), ch = m0_uni(C.h);
+	const unsigned n = (unsigned)w * (unsigned)h, nc = (unsigned)cw * (unsigned)ch;
+	M0Strip<UP, EVEN> S;
+	S.template clear<0>();
+	S.code = m0_buf(L.code, n);
+	S.b = m0_buf(L.b, 4 * n);
+	S.zd = m0_buf(L.zd, 4 * n);
+	S.out = m0_buf(L.z, 4 * n);
+	S.cc = m0_buf(UP ? C.z : C.b, 4 * nc);
+	S.lut = lut;
+	S.w = (unsigned)w;
+	S.h = (unsigned)h;
+	S.cw = (unsigned)cw;
+	S.ch = (unsigned)ch;
+	S.jt = t4.z - M0_HALO;
+	// bytes of the lane's codes, b / zd / ce to load, z and coarse b to store
+	// (an odd width's last column: loads of the pair one column to the left,
+	// of which it is the right cell, and a store of its own)
+	const bool ok = i0 >= 0 && i0 < w;
+	const bool mine = threadIdx.x >= M0_HALO / 2 && threadIdx.x < (M0_HALO + M0_TX) / 2 && ok;
+	S.lone = !EVEN && i0 == w - 1;
+	S.sh = S.lone ? 8u : 0u;
+	const unsigned il = (unsigned)(i0 - (S.lone ? 1 : 0));
+	S.vc = ok ? il : M0_OFF;
+	S.vb = ok ? 4u * il : M0_OFF;
+	S.vo = mine && !S.lone ? 4u * (unsigned)i0 : M0_OFF;
+	S.vl = mine && S.lone ? 4u * (unsigned)i0 : M0_OFF;
+	S.mine = mine;
+	S.vk = ok ? 4u * (unsigned)(i0 >> 1) : M0_OFF;
+	S.vko = mine ? 4u * (unsigned)(i0 >> 1) : M0_OFF;
+	S.wc = wc;
+	S.acc = S.tot = 0;
+	S.ca = 0.0f;
+	const int rows = h - t4.z < M0_TY ? h - t4.z : M0_TY;
+	const int steps = ((rows + 3) & ~3) + 2 * M0_HALO;
+	S.template first<0>();
+	S.template first_rows<0>();
+	S.template decode<0>();
+	for (int t = 0;; t += M0_U) {
+		if (!S.template steps4<0>(t, steps)) break;
+		if (!S.template steps4<4>(t + 4, steps)) break;
+		if (!S.template steps4<8>(t + 8, steps)) break;
+		if (!S.template steps4<12>(t + 12, steps)) break;
+		if (!S.template steps4<16>(t + 16, steps)) break;
+		if (!S.template steps4<20>(t + 20, steps)) break;
+	}
+	if constexpr (UP) {
+		double v = S.mine ? S.tot + S.acc : 0.0;
+		for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+		if (threadIdx.x == 0) tpart[tb] = v;
 	}
 }
 
@@ -2028,6 +2349,15 @@ static void with_geo(int geo, F &&f)
 	with_geo_from<Geo, 0, N>(geo, f);
 }
 
+// level 0 by strips, down or up
+template <bool UP>
+static void launch_strips(const Cg32Batch &B, hipStream_t s)
+{
+	auto k = B.odd0 ? k_mg0_strip<UP, false> : k_mg0_strip<UP, true>;
+	k<<<B.ntiles0, 64, 0, s>>>(B.tiles0, B.mg[0].lv, B.mg[0].coarse, B.scal, B.wc,
+			B.tpart);
+}
+
 static void vcycle(const Cg32Batch &B, hipStream_t s)
 {
 	const int L = B.nlev;
@@ -2036,6 +2366,9 @@ static void vcycle(const Cg32Batch &B, hipStream_t s)
 	// zd and a quarter coarse b (10 B); up reads zd, b, the code and a
 	// quarter coarse z, writes z (14 B)
 	if (B.prof) B.prof("mg_down0", 1, 0, s);
+	if (B.strips0)
+		launch_strips<false>(B, s);
+	else
 	with_geo<GeoF, MG_NFINE>(B.geo0, [&](auto g) {
 		using G = decltype(g);
 		k_mg_down<Lev0, G><<<B.ntiles0, G::T, 0, s>>>(B.tiles0, B.mg[0].lv,
@@ -2110,6 +2443,9 @@ static void vcycle(const Cg32Batch &B, hipStream_t s)
 		}
 	}
 	if (B.prof) B.prof("mg_up0", 1, 0, s);
+	if (B.strips0)
+		launch_strips<true>(B, s);
+	else
 	with_geo<GeoF, MG_NFINE>(B.geo0, [&](auto g) {
 		using G = decltype(g);
 		k_mg_up<Lev0, G, true><<<B.ntiles0, G::T, 0, s>>>(B.tiles0, B.mg[0].lv,

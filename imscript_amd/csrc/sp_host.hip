@@ -221,6 +221,26 @@ static int mg_geo_of(int l, double cells)
 	return cells >= (double)(1 << 19) ? 4 : 5;
 }
 
+// Level 0 by one wave per tile, or (0) by work-groups: the same tiles and
+// bits.  A wave is slower on its tile than 16 waves are, but 16 times as
+// many tiles run at once, with fewer operations and no barriers: strips from
+// 5e6 pixels (all planes of the batch).  Guided fills to 5e-6, us, tiles /
+// strips: 1 x 1024^2 1321 / 1480, 1 x 2048^2 1640 / 1676; 3 x 2048^2 to
+// 1e-6 3467 / 3183, 3 x 4096^2 7841 / 6935.  Tiles also where a shape was
+// chosen, where a plane's byte offsets would meet the strips' out-of-range
+// offset, and for planes one pixel wide (diagonals below 2).
+static int mg_strips(const std::vector<Cg32Plane> &cp)
+{
+	if (g_mg_geo[0] >= 0) return 0;
+	double px = 0;
+	for (const Cg32Plane &c : cp) {
+		const double n = (double)c.w * c.h;
+		if (n > (double)(1 << 30) - 1024 || c.w < 2 || c.h < 2) return 0;
+		px += n;
+	}
+	return px >= 5e6;
+}
+
 static int ensure_device()
 {
 	static std::mutex mu;
@@ -1542,6 +1562,9 @@ static int mg_plan(Plan &pl, std::vector<Cg32Plane> &cp, int bilap,
 	TRY(pl.upload(&B.tiles0, tiles0));
 	B.ntiles0 = (int)tiles0.size();
 	B.geo0 = mg_geo_of(0, 0.0);
+	B.strips0 = mg_strips(cp);
+	B.odd0 = 0;
+	for (const Cg32Plane &c : cp) B.odd0 |= c.w & 1;
 	TRY(pl.alloc(&B.tpart, tiles0.size()));
 	B.mg = mgw.data();
 	B.nlev = nlev;
