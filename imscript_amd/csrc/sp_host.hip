@@ -2156,7 +2156,10 @@ static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 		ch = (int)ceil(ch / 2.0);
 		sc--;
 	}
-	std::vector<int> key = {w, h, pd, (int)shp.size(), P.niter, (int)P.ponlit};
+	int step;   // the sweeps' step, by its bits
+	static_assert(sizeof step == sizeof P.tstep, "");
+	memcpy(&step, &P.tstep, sizeof step);
+	std::vector<int> key = {w, h, pd, (int)shp.size(), P.niter, (int)P.ponlit, step};
 	if (g_as && g_as->key == key) { *out = g_as; return SP_OK; }
 	delete g_as;
 	g_as = nullptr;
