@@ -44,11 +44,11 @@ PEAK_HBM_GBPS = 8000.0
 # measured on: TRAFFIC_SRC is the SHA-256 prefix of imscript_amd/csrc/sp_cg.hip
 # then, and the line reports traffic null when the source differs.
 TRAFFIC_PMC = {
-    "mg_up0": 633.9e6,
-    "mg_down0": 495.3e6,
-    "k32_dirspmv": 703.3e6,
+    "mg_up0": 554.9e6,
+    "mg_down0": 362.4e6,
+    "k32_dirspmv": 703.2e6,
 }
-TRAFFIC_SRC = "53d9b747b6fcb701"
+TRAFFIC_SRC = "a4df540fb588e47d"
 
 
 def kernel_source_id(name="sp_cg.hip"):
@@ -767,6 +767,9 @@ def run_amle(a):
                                    f" (tile {shape} = BIxBJxBT: BT raster sweeps fused "
                                    "per pass, one launch per wavefront of skewed tiles)"
                                    if not gs_flow() else
+                                   "k_ss_run (streaming bands of 64 skewed rows, all "
+                                   "sweeps in one launch)" if nn == 4
+                                   and "SIMPOIS_HIP_AMLE_VARIANT" not in os.environ else
                                    f"k_amle_flow<{'4-neighbour' if nn == 4 else 'table'}> "
                                    f"(tile {shape} = BIxBJxBT: BT raster sweeps fused per "
                                    "pass; one launch per pass, each skewed tile started "
@@ -1073,6 +1076,11 @@ def run_c2(a, method, full):
     # average
     ms_, n_, _ = kern["k32_dirspmv"]
     kern["k32_dirspmv"] = (ms_, n_, 27.0 * hole_frac * a.size * a.size * a.channels * n_)
+    # level 0 by strips: the code and the coarse value of every pixel (2 B);
+    # per unknown b read and zd written (down), b and zd read and z written (up)
+    for k, by in (("mg_down0", 8.0), ("mg_up0", 12.0)):
+        kern[k] = kern[k][:2] + ((2.0 + by * hole_frac) * a.size * a.size * a.channels
+                                 * kern[k][1],)
 
     mpix = a.size * a.size * a.channels / 1e6
     result = {
@@ -1142,9 +1150,9 @@ def run_c2(a, method, full):
         ms, n, by = kern[dom]
         achieved = by / (ms * 1e-3) / 1e9
         result["roofline"] = {
-            "kernel": {"mg_up0": "k_mg_up0 (fused level-0 coarse correction + "
+            "kernel": {"mg_up0": "k_mg0_strip (level-0 coarse correction + "
                                  "10 red-black half sweeps + r.z)",
-                       "mg_down0": "k_mg_down0 (fused level-0 10 red-black half "
+                       "mg_down0": "k_mg0_strip (level-0 10 red-black half "
                                    "sweeps + residual + restriction)",
                        "k32_dirspmv": "k32_dirspmv (fused CG direction + "
                                       "operator product + p.q)"}[dom],
@@ -1176,10 +1184,13 @@ def run_c2(a, method, full):
         eff = 12.0 * a.niter * tiled_px / (gs_ms * 1e-3) / 1e9
         tune = sp.autotune_report().strip().splitlines()
         finest = max(tune, key=lambda ln: int(ln.split("px=")[1].split()[0])) if tune else ""
+        # without a tuned choice the library takes the streaming bands
         shape = ([c[1:].split(":")[0] for c in finest.split("choice=")[1].split(",")
-                  if c.startswith("*")] or ["32x128x16"])[0] if finest else "32x128x16"
+                  if c.startswith("*")] or ["stream"])[0] if finest else "stream"
         result["roofline"] = {
-            "kernel": (f"k_gs_flow<1> (tile {shape} = BIxBJxBT: BT lexicographic "
+            "kernel": ("k_ss_run (streaming bands of 64 skewed rows, all sweeps of a "
+                       "level in one launch)" if gs_flow() and shape == "stream" else
+                       f"k_gs_flow<1> (tile {shape} = BIxBJxBT: BT lexicographic "
                        "sweeps fused per pass; one launch per level, each skewed "
                        "tile started once its predecessors have stored)" if gs_flow() else
                        f"k_gs_tile<1> (tile {shape} = BIxBJxBT: BT lexicographic "

@@ -1749,10 +1749,10 @@ void k_mg_up(const int4 *tiles, const MgLevel *lv,
 // 3 x 4096 x 4096, half of it unknown, a launch: down 106 us, up 127 us; by
 // the tile kernels 176 and 198.  With neither loads nor stores the launches
 // take 77 and 71 us (the operations: 2.5 cycles for a plain one, 4.4 for a
-// DPP one), without the stores alone 79 and 98: what is left over them is
-// the stores, 155 MB in short rows.  The depth of the loads (2 to 8 rows), the
-// height of a strip (44 to 132 rows: less halo, fewer waves) and leaving out
-// rows without an unknown in flight measured the same or slower.
+// DPP one); the traffic with the halo is about 70 and 105 us at a copy's
+// rate.  The depth of the loads (2 to 8 rows), taller strips (64 to 132 rows:
+// less halo, fewer waves) and leaving out rows without an unknown in flight
+// measured the same or slower.
 constexpr int M0_NU = 5, M0_HALO = 2 * M0_NU, M0_TX = 128 - 2 * M0_HALO, M0_U = 24;
 constexpr int M0_TY = MG_FINE_TY[MG_STRIP_GEO];
 constexpr int M0_BA = 4, M0_CA = 7;      // rows that b / codes are ahead
