@@ -26,6 +26,7 @@
 #include <list>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 // ------------------------------------------------------------- errors
@@ -1897,8 +1898,11 @@ extern "C" void sp_plan_cache_limit(int max_plans, size_t max_bytes)
 	cache_trim(nullptr, g_cache_max, g_cache_max_bytes);
 }
 
+static void hc_clear();
+
 extern "C" void sp_plan_cache_clear(void)
 {
+	hc_clear();
 	std::lock_guard<std::mutex> lk(g_cache_mu);
 	cache_trim(nullptr, 0, 0);
 }
@@ -2044,6 +2048,100 @@ extern "C" int sp_solve_device(float *d_out, const float *d_in, const float *d_d
 	return sp_solve_batch_device(1, &I, p, stream, st);
 }
 
+// Copies between the caller's pageable memory and the device.  A plain
+// hipMemcpy passes such memory through one thread (and takes the page faults
+// of a fresh result there); large copies go in chunks by up to HC_THREADS
+// threads, each through a pinned buffer of its own, so the host's copies
+// overlap with each other and with the transfers.  The buffers are kept for
+// the next call, at most HC_THREADS of them in the process, and freed with
+// the plan cache; a call that finds none free copies plainly.  A fill of
+// 3 x 2159 x 3839 host arrays (100 MB each way): 17.2 -> 8.9 ms.  Below
+// HC_MIN a copy takes under 1.5 ms and the threads are not worth starting.
+constexpr size_t HC_CHUNK = 4 << 20, HC_MIN = 16 << 20;
+constexpr int HC_THREADS = 4;
+static std::mutex g_hc_mu;
+static std::vector<void *> g_hc_free;
+static int g_hc_made;
+
+static void *hc_take()
+{
+	{
+		std::lock_guard<std::mutex> lk(g_hc_mu);
+		if (!g_hc_free.empty()) {
+			void *p = g_hc_free.back();
+			g_hc_free.pop_back();
+			return p;
+		}
+		if (g_hc_made >= HC_THREADS) return nullptr;
+		g_hc_made++;
+	}
+	void *p = nullptr;
+	if (hipHostMalloc(&p, HC_CHUNK, hipHostMallocPortable) == hipSuccess) return p;
+	(void)hipGetLastError();
+	std::lock_guard<std::mutex> lk(g_hc_mu);
+	g_hc_made--;
+	return nullptr;
+}
+
+static void hc_give(void *p)
+{
+	std::lock_guard<std::mutex> lk(g_hc_mu);
+	g_hc_free.push_back(p);   // (room reserved by hc_copy)
+}
+
+static void hc_clear()
+{
+	std::lock_guard<std::mutex> lk(g_hc_mu);
+	for (void *p : g_hc_free) (void)hipHostFree(p);
+	g_hc_made -= (int)g_hc_free.size();
+	g_hc_free.clear();
+}
+
+static hipError_t hc_copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind)
+{
+	int dev = 0;
+	if (bytes < HC_MIN || hipGetDevice(&dev) != hipSuccess)
+		return hipMemcpy(dst, src, bytes, kind);
+	void *slot[HC_THREADS] = {};
+	std::thread th[HC_THREADS];
+	int ns = 0;
+	{
+		std::lock_guard<std::mutex> lk(g_hc_mu);
+		try { g_hc_free.reserve(HC_THREADS); } catch (...) { ns = -1; }
+	}
+	if (ns < 0) return hipMemcpy(dst, src, bytes, kind);
+	while (ns < HC_THREADS && (slot[ns] = hc_take())) ns++;
+	if (!ns) return hipMemcpy(dst, src, bytes, kind);
+	std::atomic<size_t> next{0};
+	std::atomic<int> err{(int)hipSuccess};
+	const bool up = kind == hipMemcpyHostToDevice;
+	auto run = [&](void *buf) {
+		for (;;) {
+			const size_t o = next.fetch_add(HC_CHUNK);
+			if (o >= bytes || err.load() != (int)hipSuccess) return;
+			const size_t n = std::min(HC_CHUNK, bytes - o);
+			if (up) memcpy(buf, (const char *)src + o, n);
+			const hipError_t e = up ? hipMemcpy((char *)dst + o, buf, n, kind)
+				: hipMemcpy(buf, (const char *)src + o, n, kind);
+			if (e != hipSuccess) { err.store((int)e); return; }
+			if (!up) memcpy((char *)dst + o, buf, n);
+		}
+	};
+	for (int k = 1; k < ns; k++)
+		try {
+			th[k] = std::thread([&run, dev, b = slot[k]] {
+				if (hipSetDevice(dev) == hipSuccess) run(b);
+			});
+		} catch (...) {
+			break;   // fewer threads
+		}
+	run(slot[0]);
+	for (int k = 1; k < ns; k++)
+		if (th[k].joinable()) th[k].join();
+	for (int k = 0; k < ns; k++) hc_give(slot[k]);
+	return (hipError_t)err.load();
+}
+
 extern "C" int sp_solve_host(float *out, const float *in, const float *dat,
 		int w, int h, int pd, const sp_params *p, sp_stats *st)
 {
@@ -2061,11 +2159,11 @@ extern "C" int sp_solve_host(float *out, const float *in, const float *dat,
 		cleanup();
 		return set_err(SP_ERR_NOMEM, "device allocation of %zu bytes failed", n * 4);
 	}
-	if (hipMemcpy(d_in, in, n * 4, hipMemcpyHostToDevice) != hipSuccess
-			|| (dat && hipMemcpy(d_dat, dat, n * 4, hipMemcpyHostToDevice) != hipSuccess))
+	if (hc_copy(d_in, in, n * 4, hipMemcpyHostToDevice) != hipSuccess
+			|| (dat && hc_copy(d_dat, dat, n * 4, hipMemcpyHostToDevice) != hipSuccess))
 		rc = set_err(SP_ERR_HIP, "upload failed");
 	if (!rc) rc = sp_solve_device(d_out, d_in, d_dat, w, h, pd, p, nullptr, st);
-	if (!rc && hipMemcpy(out, d_out, n * 4, hipMemcpyDeviceToHost) != hipSuccess)
+	if (!rc && hc_copy(out, d_out, n * 4, hipMemcpyDeviceToHost) != hipSuccess)
 		rc = set_err(SP_ERR_HIP, "download failed");
 	cleanup();
 	return rc;
