@@ -480,6 +480,8 @@ struct Plan {
 	std::vector<std::pair<void *, size_t>> allocs;
 	size_t bytes = 0;                // device bytes held by allocs
 	int *d_cnt = nullptr;
+	spk::CountWork *d_count = nullptr;   // of every level's members, finest level first
+	int ncount = 0;
 	float **d_outs = nullptr;
 	// FP64 CG scratch, sized for the largest plane
 	float *cg_q = nullptr;
@@ -1035,6 +1037,7 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 		TRY(pl.upload(&pl.d_outs, outs));
 	}
 	size_t cnt_off = 0;
+	std::vector<spk::CountWork> cw;
 	for (int k = 0; k < nlev; k++) {
 		LevelPlan &L = pl.lv[k];
 		const int nm = (int)L.members.size();
@@ -1083,6 +1086,8 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 		TRY(pl.upload(&L.d_bw, bw));
 		TRY(pl.upload(&L.d_first, first));
 		TRY(pl.alloc(&L.d_bcnt, bw.size()));
+		for (int m = 0; m < nm; m++)
+			cw.push_back({L.sp[m].cnt, L.d_bcnt + first[m], first[m + 1] - first[m]});
 		// PONLIT restricts the work to the level of that width (:272-273)
 		L.nsweep.assign(nm, std::max(P.niter, 0));
 		L.cgit.assign(nm, P.cgit);
@@ -1159,6 +1164,8 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 		TRY(ss_level(pl, L, has_f));
 		if (!L.ss.nt || P.autotune) TRY(gs_build(pl, L, gs_default_var(pl.R)));
 	}
+	TRY(pl.upload(&pl.d_count, cw));
+	pl.ncount = (int)cw.size();
 	// parent (finer) and coarse descriptors aligned with each level's members
 	for (int k = 0; k < nlev; k++) {
 		LevelPlan &L = pl.lv[k];
@@ -1792,13 +1799,12 @@ static int plan_execute(Plan &pl, hipStream_t s, sp_stats *st)
 		ProfScope pr("pyramid", s);
 		LevelPlan &L0 = pl.lv[0];
 		spk::launch_prepare(L0.d_sp, L0.d_bw, L0.nbw, L0.d_bcnt, s);
-		spk::launch_count(L0.d_sp, (int)L0.members.size(), L0.d_first, L0.d_bcnt, s);
 		for (int k = 1; k < nlev; k++) {
 			LevelPlan &L = pl.lv[k];
 			spk::launch_restrict(L.d_parent, L.d_sp, L.d_bw, L.nbw, pl.P.pmsfac,
 					L.d_bcnt, s);
-			spk::launch_count(L.d_sp, (int)L.members.size(), L.d_first, L.d_bcnt, s);
 		}
+		spk::launch_count(pl.d_count, pl.ncount, s);
 		HIPCHK(hipGetLastError());
 	}
 	// coarse to fine
@@ -3180,7 +3186,7 @@ static int cg_extend_host(float *out, const float *in, const float *dat, int w,
 	hipStream_t s = nullptr;
 	LevelPlan &L0 = pl.lv[0];
 	spk::launch_prepare(L0.d_sp, L0.d_bw, L0.nbw, L0.d_bcnt, s);
-	spk::launch_count(L0.d_sp, 1, L0.d_first, L0.d_bcnt, s);
+	spk::launch_count(pl.d_count, 1, s);
 	TRY(run_cg64(pl, 0, 0, maxit, bilap, eps, s));
 	// :251-256 and the nmask == 0 branch :203-207
 	int nmask = 0;

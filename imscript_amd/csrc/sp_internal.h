@@ -205,8 +205,8 @@ void launch_prepare(const SpPlane *planes, const BlockWork *bw, int nblocks,
 		int *bcnt, hipStream_t s);
 void launch_restrict(const SpPlane *fine, const SpPlane *coarse,
 		const BlockWork *bw, int nblocks, double pmsfac, int *bcnt, hipStream_t s);
-void launch_count(const SpPlane *planes, int nplanes, const int *first,
-		const int *bcnt, hipStream_t s);
+struct CountWork { int *cnt; const int *bcnt; int n; };
+void launch_count(const CountWork *cw, int n, hipStream_t s);
 void launch_init(const SpPlane *lv, const SpPlane *coarse, const BlockWork *bw,
 		int nblocks, hipStream_t s);
 void launch_finalize(const SpPlane *lv, float *const *outs,
