@@ -2211,8 +2211,9 @@ static AdjScratch *g_adj = nullptr;
 //   turned by 180 degrees a backward sweep is a forward one, and
 //   (I/t + U)^-1 lambda is one forward sweep from 0 with data -lambda: the
 //   library's own Gauss-Seidel kernels run both (boundary 0 at the known
-//   pixels, data 0 after the first), one sweep at a time so that each
-//   nu_j is added up.
+//   pixels, data 0 after the first), in one run that adds up every nu_j
+//   (one sweep at a time where neither of the summing kernels takes the
+//   level).
 // * The initial value at the holes is the bilinear x2 of the coarser
 //   level's output (simpois.c:199-239): its transpose gives the coarser
 //   level's v, and the recursion goes on there.
