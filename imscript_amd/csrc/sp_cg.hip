@@ -16,6 +16,7 @@
 // Planes that have converged are skipped by all later launches.
 #include "sp_internal.h"
 #include "sp_cg.h"
+#include "sp_strip.h"
 #include "../../include/simpois_hip.h"
 
 namespace spk {
@@ -1753,13 +1754,10 @@ void k_mg_up(const int4 *tiles, const MgLevel *lv,
 // rate.  The depth of the loads (2 to 8 rows), taller strips (64 to 132 rows:
 // less halo, fewer waves) and leaving out rows without an unknown in flight
 // measured the same or slower.
-constexpr int M0_NU = 5, M0_HALO = 2 * M0_NU, M0_TX = 128 - 2 * M0_HALO, M0_U = 24;
-constexpr int M0_TY = MG_FINE_TY[MG_STRIP_GEO];
-constexpr int M0_BA = 4, M0_CA = 7;      // rows that b / codes are ahead
-constexpr unsigned M0_OFF = 0xfffffff0u; // beyond every buffer
+constexpr int M0_U = 24;
 static_assert(M0_CA + 2 * M0_NU + 1 < M0_U, "ring too short");
 static_assert(M0_TX == MG_FINE_TX[MG_STRIP_GEO] && M0_NU == MG_FINE_NU[MG_STRIP_GEO]
-		&& M0_TY % 4 == 0, "strips are the default tiles");
+		&& M0_TY == MG_FINE_TY[MG_STRIP_GEO] && M0_TY % 4 == 0, "strips are the default tiles");
 
 constexpr int m0_at(int k) { return (k + 2 * M0_U) % M0_U; }
 
@@ -1774,14 +1772,14 @@ static __device__ __forceinline__ float m0_east(float v)   // lane + 1
 }
 
 // A buffer's descriptor.  Addresses are a lane's byte offset in the row (a
-// register that does not change, or M0_OFF) plus the row's (scalar); a row
-// that is not to be touched has a descriptor of 0 bytes.
+// register that does not change, or M0_OFF) plus the row's (scalar), which
+// sp_strip.h gives.
 struct M0Buf {
 	uintptr_t p;
 	unsigned n;
-	__device__ __forceinline__ __amdgpu_buffer_rsrc_t row(bool in) const
+	__device__ __forceinline__ __amdgpu_buffer_rsrc_t desc(M0Row r) const
 	{
-		return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, in ? (int)n : 0, 0x00020000);
+		return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)r.n, 0x00020000);
 	}
 };
 
@@ -1800,42 +1798,37 @@ template <bool UP, bool EVEN> struct M0Strip {
 	unsigned cd[M0_U], dg[UP ? 1 : M0_U];   // codes; diagonals, a byte each
 	M0Buf code, b, zd, out, cc;
 	const float *lut;                // rdiag of a code byte (LDS)
-	unsigned vc, vb, vo, vl, vk, vko;   // the lane's offsets (see kernel)
-	bool mine, lone;                  // odd width: the pair is the last column alone
-	unsigned sh;                     // its code's shift
-	unsigned w, h, cw, ch;
-	int jt;                          // image row of strip row 0
+	M0Lane ln;                       // the lane's offsets
+	unsigned sh;                     // the code's shift of a lone last column
+	M0Rows rows;
 	float wc, ca;
 	double acc, tot;                 // r.z of four rows, of the rows before them
 
-	__device__ __forceinline__ bool row_in(int r) const { return (unsigned)(jt + r) < h; }
-	// the row's first pixel; outside the image, where no lane touches any, that
-	// of the nearest row: a scalar offset never exceeds its buffer
-	__device__ __forceinline__ unsigned row_at(int r) const
-	{ return (unsigned)clampi(jt + r, 0, (int)h - 1) * w; }
-	__device__ __forceinline__ unsigned coarse_at(int r) const
-	{ return (unsigned)clampi((jt + r) >> 1, 0, (int)ch - 1) * cw; }
 	template <int K> __device__ __forceinline__ void load_code(int r)
 	{
-		const __amdgpu_buffer_rsrc_t d = code.row(row_in(r));
-		cd[K] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(d, vc, row_at(r), 0);
+		const M0Row at = rows.code(r, code.n);
+		cd[K] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(code.desc(at), ln.vc,
+				at.at, 0);
 	}
 	template <int K> __device__ __forceinline__ void load_row(int r)
 	{
 		if constexpr (!EVEN) cd[K] >>= sh;
-		const unsigned o = cd[K] ? vb : M0_OFF, at = 4u * row_at(r);
+		const unsigned o = cd[K] ? ln.vb : M0_OFF;
+		const M0Row at = rows.values(r, b.n);
 		const gu2 v = __builtin_bit_cast(gu2,
-				__builtin_amdgcn_raw_buffer_load_b64(b.row(true), o, at, 0));
+				__builtin_amdgcn_raw_buffer_load_b64(b.desc(at), o, at.at, 0));
 		b0[K] = __uint_as_float(v.x);
 		b1[K] = __uint_as_float(v.y);
 		if constexpr (UP) {
 			const gu2 y = __builtin_bit_cast(gu2,
-					__builtin_amdgcn_raw_buffer_load_b64(zd.row(true), o, at, 0));
+					__builtin_amdgcn_raw_buffer_load_b64(zd.desc(at), o, at.at, 0));
 			z0[K] = __uint_as_float(y.x);
 			z1[K] = __uint_as_float(y.y);
-			if constexpr (!(K & 1))
+			if constexpr (!(K & 1)) {
+				const M0Row co = rows.coarse(r, cc.n);
 				ce[K / 2] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-						cc.row(true), vk, 4u * coarse_at(r), 0));
+						cc.desc(co), ln.vk, co.at, 0));
+			}
 		} else {
 			z0[K] = z1[K] = 0.0f;
 		}
@@ -1879,11 +1872,11 @@ template <bool UP, bool EVEN> struct M0Strip {
 		decode<m0_at(U + 1)>();
 		// row t arrives
 		if constexpr (!EVEN) {
-			b0[U] = lone ? b1[U] : b0[U];
-			b1[U] = lone ? 0.0f : b1[U];
+			b0[U] = ln.lone ? b1[U] : b0[U];
+			b1[U] = ln.lone ? 0.0f : b1[U];
 			if constexpr (UP) {
-				z0[U] = lone ? z1[U] : z0[U];
-				z1[U] = lone ? 0.0f : z1[U];
+				z0[U] = ln.lone ? z1[U] : z0[U];
+				z1[U] = ln.lone ? 0.0f : z1[U];
 			}
 		}
 		if constexpr (UP) {
@@ -1894,16 +1887,15 @@ template <bool UP, bool EVEN> struct M0Strip {
 		half<U, 0>();
 		// row t - 2 nu is finished
 		constexpr int k = m0_at(U - 2 * M0_NU), no = m0_at(k - 1), so = m0_at(k + 1);
-		const bool o = t >= 2 * M0_HALO;
-		const __amdgpu_buffer_rsrc_t d = (UP ? out : zd).row(o);
-		const unsigned at = 4u * row_at(t - M0_HALO);
+		const M0Row at = rows.out(t, out.n);
+		const __amdgpu_buffer_rsrc_t d = (UP ? out : zd).desc(at);
 		const bool any = UP ? r0[k] + r1[k] != 0.0f : dg[UP ? 0 : k] != 0u;
 		__builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(
 				decltype(__builtin_amdgcn_raw_buffer_load_b64(d, 0, 0, 0)),
-				gf2{z0[k], z1[k]}), d, any ? vo : M0_OFF, at, 0);
+				gf2{z0[k], z1[k]}), d, any ? ln.vo : M0_OFF, at.at, 0);
 		if constexpr (!EVEN)
 			__builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(z0[k]), d,
-					any ? vl : M0_OFF, at, 0);
+					any ? ln.vl : M0_OFF, at.at, 0);
 		if constexpr (UP) {
 			acc = __builtin_fma((double)b0[k], (double)z0[k], acc);
 			acc = __builtin_fma((double)b1[k], (double)z1[k], acc);
@@ -1922,9 +1914,9 @@ template <bool UP, bool EVEN> struct M0Strip {
 			ca = U & 1 ? ca + v0 : v0;
 			ca += v1;
 			if constexpr (U & 1) {
-				const bool in = o && (jt + t - M0_HALO) >> 1 < (int)ch;
-				__builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ca), cc.row(in), vko,
-						4u * coarse_at(t - M0_HALO), 0);
+				const M0Row co = rows.coarse_out(t, cc.n);
+				__builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ca), cc.desc(co), ln.vko,
+						co.at, 0);
 			}
 		}
 	}
@@ -1978,7 +1970,6 @@ void k_mg0_strip(const int4 *tiles, const MgLevel *lv, const MgLevel *coarse,
 	if (!sc[t4.x].active) return;
 #pragma unroll
 	for (int k = 0; k < 4; k++) lut[threadIdx.x + 64 * k] = Lev0::rdiag(threadIdx.x + 64 * k);
-	const int i0 = t4.y - M0_HALO + 2 * (int)threadIdx.x;
 	const int w = m0_uni(L.w), h = m0_uni(L.h), cw = m0_uni(C.w), ch = m0_uni(C.h);
 	const unsigned n = (unsigned)w * (unsigned)h, nc = (unsigned)cw * (unsigned)ch;
 	M0Strip<UP, EVEN> S;
@@ -1989,31 +1980,13 @@ void k_mg0_strip(const int4 *tiles, const MgLevel *lv, const MgLevel *coarse,
 	S.out = m0_buf(L.z, 4 * n);
 	S.cc = m0_buf(UP ? C.z : C.b, 4 * nc);
 	S.lut = lut;
-	S.w = (unsigned)w;
-	S.h = (unsigned)h;
-	S.cw = (unsigned)cw;
-	S.ch = (unsigned)ch;
-	S.jt = t4.z - M0_HALO;
-	// bytes of the lane's codes, b / zd / ce to load, z and coarse b to store
-	// (an odd width's last column: loads of the pair one column to the left,
-	// of which it is the right cell, and a store of its own)
-	const bool ok = i0 >= 0 && i0 < w;
-	const bool mine = threadIdx.x >= M0_HALO / 2 && threadIdx.x < (M0_HALO + M0_TX) / 2 && ok;
-	S.lone = !EVEN && i0 == w - 1;
-	S.sh = S.lone ? 8u : 0u;
-	const unsigned il = (unsigned)(i0 - (S.lone ? 1 : 0));
-	S.vc = ok ? il : M0_OFF;
-	S.vb = ok ? 4u * il : M0_OFF;
-	S.vo = mine && !S.lone ? 4u * (unsigned)i0 : M0_OFF;
-	S.vl = mine && S.lone ? 4u * (unsigned)i0 : M0_OFF;
-	S.mine = mine;
-	S.vk = ok ? 4u * (unsigned)(i0 >> 1) : M0_OFF;
-	S.vko = mine ? 4u * (unsigned)(i0 >> 1) : M0_OFF;
+	S.rows = {(unsigned)w, (unsigned)h, (unsigned)cw, (unsigned)ch, t4.z - M0_HALO};
+	S.ln = m0_lane<EVEN>((int)threadIdx.x, t4.y, w);
+	S.sh = S.ln.lone ? 8u : 0u;
 	S.wc = wc;
 	S.acc = S.tot = 0;
 	S.ca = 0.0f;
-	const int rows = h - t4.z < M0_TY ? h - t4.z : M0_TY;
-	const int steps = ((rows + 3) & ~3) + 2 * M0_HALO;
+	const int steps = m0_steps(h, t4.z);
 	S.template first<0>();
 	S.template first_rows<0>();
 	S.template decode<0>();
@@ -2026,7 +1999,7 @@ void k_mg0_strip(const int4 *tiles, const MgLevel *lv, const MgLevel *coarse,
 		if (!S.template steps4<20>(t + 20, steps)) break;
 	}
 	if constexpr (UP) {
-		double v = S.mine ? S.tot + S.acc : 0.0;
+		double v = S.ln.mine ? S.tot + S.acc : 0.0;
 		for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
 		if (threadIdx.x == 0) tpart[tb] = v;
 	}
