@@ -629,6 +629,19 @@ static int gs_tiles(const Plan &pl, const LevelPlan &L, int var,
 	return SP_OK;
 }
 
+// the word that a dependence wait sets when it gives up, and its host copy
+// (a plan may share another's device word: it has no copy then)
+static int gs_err_ensure(Plan &pl)
+{
+	if (pl.gs_err) return SP_OK;
+	TRY(pl.alloc(&pl.gs_err, 1));
+	HIPCHK(hipMemset(pl.gs_err, 0, sizeof(int)));
+	if (hipHostMalloc(&pl.h_gs_err, sizeof(int)) != hipSuccess)
+		return set_err(SP_ERR_NOMEM, "pinned host allocation of 4 bytes failed");
+	*pl.h_gs_err = 0;
+	return SP_OK;
+}
+
 // the dependence-ordered launch's data for the tiles of variant var: each
 // member's tile grid and one flag per grid cell, 0 for a tile (below every
 // epoch), INT_MAX where the grid has no tile (never waited for); *d_flags
@@ -654,13 +667,7 @@ static int gs_flow_build(Plan &pl, const LevelPlan &L, int var,
 	TRY(pl.upload(d_fi, fi));
 	TRY(pl.upload(d_flags, flags));
 	if (!pl.gs_claim) TRY(pl.alloc(&pl.gs_claim, 1));
-	if (!pl.gs_err) {
-		TRY(pl.alloc(&pl.gs_err, 1));
-		HIPCHK(hipMemset(pl.gs_err, 0, sizeof(int)));
-		if (hipHostMalloc(&pl.h_gs_err, sizeof(int)) != hipSuccess)
-			return set_err(SP_ERR_NOMEM, "pinned host allocation of 4 bytes failed");
-	}
-	return SP_OK;
+	return gs_err_ensure(pl);
 }
 
 static int gs_build(Plan &pl, LevelPlan &L, int var)
@@ -760,12 +767,7 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bo
 	TRY(pl.upload(&ss.d_inst, in));
 	TRY(pl.upload(&ss.d_tasks, tl));
 	TRY(pl.upload(&ss.d_bw, bw));
-	if (!pl.gs_err) {
-		TRY(pl.alloc(&pl.gs_err, 1));
-		HIPCHK(hipMemset(pl.gs_err, 0, sizeof(int)));
-		if (hipHostMalloc(&pl.h_gs_err, sizeof(int)) != hipSuccess)
-			return set_err(SP_ERR_NOMEM, "pinned host allocation of 4 bytes failed");
-	}
+	TRY(gs_err_ensure(pl));
 	ss.inst = in;
 	ss.nprog = (int)nprog;
 	// values stay small in averages: AMLE's, and the sweeps' for t <= 1/4
@@ -2250,6 +2252,20 @@ struct AsScratch {
 };
 static std::mutex g_as_mu;
 static AsScratch *g_as = nullptr;
+// error word of the dependence waits of every sweep of a gradient (gs_err /
+// h_gs_err of this object, which lives as long as the process): the images of
+// one call may each replace the scratch, and the call reads the word once
+static Plan *g_as_err = nullptr;
+
+static int as_err_ensure()
+{
+	if (g_as_err) return SP_OK;
+	Plan *E = new Plan;
+	int rc = gs_err_ensure(*E);
+	if (rc) { delete E; return rc; }
+	g_as_err = E;
+	return SP_OK;
+}
 
 static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 {
@@ -2299,6 +2315,7 @@ static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 			planes.push_back(PlaneIn{L.w, L.h, L.g_rot + L.n * l, L.f_rot + L.n * l,
 				L.u_rot + L.n * l});
 		L.sweep = new Plan;
+		L.sweep->gs_err = g_as_err->gs_err;
 		rc = plan_create(*L.sweep, planes, P1, true);
 		if (rc) break;
 		// the summing sweeps hold the values after each of them: at most
@@ -2310,6 +2327,7 @@ static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 			P2.niter = part ? L.nsweep % L.group : L.group;
 			if (!P2.niter) break;
 			Plan *pl = new Plan;
+			pl->gs_err = g_as_err->gs_err;
 			(part ? L.rest : L.sum) = pl;
 			for (int l = 0; l < pd; l++) pl->acc.push_back(L.acc + L.n * l);
 			rc = plan_create(*pl, planes, P2, false);
@@ -2412,21 +2430,30 @@ static int adjoint_sweeps(int n, const sp_adjoint_image *imgs, const sp_params &
 		return set_err(SP_ERR_ARG, "the adjoint takes the data term itself "
 				"(guidance = 0); differentiate plambda's Laplacian separately");
 	std::lock_guard<std::mutex> lk(g_as_mu);
+	TRY(as_err_ensure());
 	hipEvent_t e0, e1;
 	HIPCHK(hipEventCreate(&e0));
 	HIPCHK(hipEventCreate(&e1));
 	HIPCHK(hipEventRecord(e0, s));
-	int levels = 0;
-	for (int i = 0; i < n; i++) {
-		const int rc = adjoint_sweeps_image(imgs[i], P, s, &levels);
-		if (rc) { (void)hipEventDestroy(e0); (void)hipEventDestroy(e1); return rc; }
-	}
-	HIPCHK(hipEventRecord(e1, s));
-	HIPCHK(hipEventSynchronize(e1));
+	int levels = 0, rc = SP_OK;
+	for (int i = 0; i < n && !rc; i++) rc = adjoint_sweeps_image(imgs[i], P, s, &levels);
+	// a wait that gave up left wrong values
+	(void)hipMemcpyAsync(g_as_err->h_gs_err, g_as_err->gs_err, sizeof(int),
+			hipMemcpyDeviceToHost, s);
+	(void)hipEventRecord(e1, s);
+	if (hipEventSynchronize(e1) != hipSuccess && !rc)
+		rc = set_err(SP_ERR_HIP, "gradient of the sweeps failed");
 	float ms = 0;
 	(void)hipEventElapsedTime(&ms, e0, e1);
 	(void)hipEventDestroy(e0);
 	(void)hipEventDestroy(e1);
+	if (*g_as_err->h_gs_err) {
+		*g_as_err->h_gs_err = 0;
+		(void)hipMemset(g_as_err->gs_err, 0, sizeof(int));
+		if (!rc) rc = set_err(SP_ERR_HIP, "dependence wait timed out in the gradient of "
+				"the sweeps");
+	}
+	TRY(rc);
 	if (st) { st->levels = levels; st->cg_iters_finest = 0; st->elapsed_ms = ms; }
 	return SP_OK;
 }
@@ -2591,7 +2618,6 @@ static int amle_build(AmlePlan &A, int T)
 		TRY(ss_build(A.mem, sc.ss, in, spk::SS_AMLE));
 		if (sc.ss.nt) {
 			sc.px = (long)ninst * T * A.w * A.h;
-			*A.mem.h_gs_err = 0;
 			A.sched.push_back(sc);
 			return SP_OK;
 		}
@@ -2625,13 +2651,7 @@ static int amle_build(AmlePlan &A, int T)
 			sc.nblocks = std::min(sc.ntiles, spk::amle_flow_blocks(A.R, A.var,
 					A.nn == 4 && (A.w > 1 || A.h > 1)));
 			if (!A.mem.gs_claim) TRY(A.mem.alloc(&A.mem.gs_claim, 1));
-			if (!A.mem.gs_err) {
-				TRY(A.mem.alloc(&A.mem.gs_err, 1));
-				HIPCHK(hipMemset(A.mem.gs_err, 0, sizeof(int)));
-				if (hipHostMalloc(&A.mem.h_gs_err, sizeof(int)) != hipSuccess)
-					return set_err(SP_ERR_NOMEM, "pinned host allocation of 4 bytes failed");
-				*A.mem.h_gs_err = 0;
-			}
+			TRY(gs_err_ensure(A.mem));
 		}
 	}
 	A.sched.push_back(sc);
