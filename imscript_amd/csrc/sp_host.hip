@@ -382,7 +382,12 @@ static int dev_alloc(void **p, size_t bytes)
 	if (cap && live + bytes > cap)
 		return set_err(SP_ERR_NOMEM, "device allocation of %zu bytes refused: the "
 				"library holds %zu of its %zu-byte cap", bytes, live, cap);
-	HIPCHK(hipMalloc(p, bytes));
+	const hipError_t e = hipMalloc(p, bytes);
+	if (e != hipSuccess) {
+		*p = nullptr;
+		(void)hipGetLastError();   // (the caller may go on with less)
+		HIPCHK(e);
+	}
 	g_live_bytes += bytes;
 	return SP_OK;
 }
@@ -522,6 +527,9 @@ struct Plan {
 	unsigned *gs_claim = nullptr;
 	int *gs_err = nullptr, *h_gs_err = nullptr;
 	bool gs_flow_used = false;
+	// whether the streaming sweeps may be used, and whether their scratch was
+	// asked for: a plan that does not fit in memory is built again without
+	bool stream = true, streamed = false;
 
 	// where each plane's values after the first sweeps are added up (the
 	// adjoint's sweeps, one level without data terms); empty: not asked for
@@ -688,10 +696,13 @@ static int gs_build(Plan &pl, LevelPlan &L, int var)
 // streaming kernel, and its data if so, in memory of pl.  It takes positive
 // steps (the coefficient marks a known pixel by a negative zero) and planes
 // whose skewed layout a 32-bit byte offset reaches.  SIMPOIS_HIP_GS_FLOW=0
-// asks for the tiles.
+// asks for the tiles.  The layouts take 2.2 times the plane's bytes at 4096 x
+// 4096, 6.7 times at 256 x 256 and more for narrow planes; where they do not
+// fit (SP_ERR_NOMEM, pl.streamed set) the caller builds the plan again with
+// pl.stream off, in tiles, which need none of it.
 static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bool sum = false)
 {
-	if (in.empty() || !g_gs_flow) return SP_OK;
+	if (in.empty() || !g_gs_flow || !pl.stream) return SP_OK;
 	int tmax = 0;
 	double px = 0;
 	for (const spk::SsInst &I : in) {
@@ -760,6 +771,7 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bo
 	// the plans of ten such calls 18 ms instead of 230
 	nbz = rup64(nbz);
 	float *pool = nullptr;
+	pl.streamed = true;
 	TRY(pl.alloc(&pool, 2 * ncell + nbz + nprog + 3 + nhist));
 	spk::launch_ss_clear(ss.op, pool, ncell, nullptr);
 	float *C = pool, *A = pool + ncell, *hist = pool + 2 * ncell, *const bz = hist + nhist;
@@ -1943,9 +1955,10 @@ extern "C" void sp_plan_cache_clear(void)
 	cache_trim(nullptr, 0, 0);
 }
 
-// the cached plan of a call (created on a miss); the caller holds g_cache_mu
+// the cached plan of a call (created on a miss, with streaming sweeps where
+// `stream` allows them); the caller holds g_cache_mu
 static int cache_get(const std::vector<PlaneIn> &planes, const sp_params &P,
-		bool has_f, int transpose, Plan **out)
+		bool has_f, int transpose, bool stream, Plan **out)
 {
 	std::vector<char> key;
 	auto put = [&](const void *v, size_t n) {
@@ -1970,9 +1983,10 @@ static int cache_get(const std::vector<PlaneIn> &planes, const sp_params &P,
 			*out = g_cache.front();
 			return SP_OK;
 		}
-	for (int attempt = 0;; attempt++) {
+	for (;;) {
 		Plan *pl = new Plan;
 		pl->transpose = transpose;
+		pl->stream = stream;
 		const int rc = plan_create(*pl, planes, P, has_f);
 		if (rc == SP_OK) {
 			pl->key = key;
@@ -1980,11 +1994,22 @@ static int cache_get(const std::vector<PlaneIn> &planes, const sp_params &P,
 			*out = pl;
 			return SP_OK;
 		}
+		const bool streamed = pl->streamed;
 		delete pl;
-		// out of device memory with plans cached: free them, try once more
-		if (rc != SP_ERR_NOMEM || attempt || g_cache.empty()) return rc;
-		cache_trim(nullptr, 0, 0);
+		// out of device memory: with plans cached free them and try once more,
+		// then without the streaming sweeps' scratch
+		if (rc != SP_ERR_NOMEM) return rc;
+		if (!g_cache.empty()) cache_trim(nullptr, 0, 0);
+		else if (streamed) stream = false;
+		else return rc;
 	}
+}
+
+// forget a cached plan; the caller holds g_cache_mu
+static void cache_drop(Plan *pl)
+{
+	g_cache.remove(pl);
+	delete pl;
 }
 
 // FP64 residual of each plane's output over its holes and the holes
@@ -2041,12 +2066,23 @@ static int solve_batch(int n, const sp_image *imgs, const sp_params *p, void *st
 	hipStream_t s = (hipStream_t)stream;
 	std::lock_guard<std::mutex> lk(g_cache_mu);
 	Plan *pl = nullptr;
-	TRY(cache_get(planes, *p, has_f, transpose, &pl));
-	const int rc = plan_execute(*pl, s, st);
+	std::vector<double> rel;
+	std::vector<int> holes;
+	auto run = [&](bool stream) {
+		TRY(cache_get(planes, *p, has_f, transpose, stream, &pl));
+		TRY(plan_execute(*pl, s, st));
+		return ps ? plane_residuals(*pl, s, rel, holes) : SP_OK;
+	};
+	int rc = run(true);
+	// the scratch of a solver built on first use did not fit beside the
+	// streaming sweeps': once more without them
+	if (rc == SP_ERR_NOMEM && pl && pl->streamed) {
+		(void)hipStreamSynchronize(s);
+		cache_drop(pl);
+		pl = nullptr;
+		rc = run(false);
+	}
 	if (rc == SP_OK && ps) {
-		std::vector<double> rel;
-		std::vector<int> holes;
-		TRY(plane_residuals(*pl, s, rel, holes));
 		for (size_t q = 0; q < planes.size(); q++) {
 			sp_plane_stats &o = ps[q];
 			o.status = pl->status_finest[q];
@@ -2059,7 +2095,7 @@ static int solve_batch(int n, const sp_image *imgs, const sp_params *p, void *st
 			if (pl->R != 3 && !std::isfinite(rel[q])) o.status = SP_PLANE_NONFINITE;
 		}
 	}
-	cache_trim(pl, g_cache_max, g_cache_max_bytes);
+	if (pl) cache_trim(pl, g_cache_max, g_cache_max_bytes);
 	return rc;
 }
 
@@ -2817,20 +2853,26 @@ extern "C" int sp_amle_device(float *d_out, const float *d_in, const float *d_in
 			A->niter != niter || A->trace != trace || A->var != var) {
 		// the old plan's scratch may still be in use on its stream
 		if (A && A->used) HIPCHK(hipEventSynchronize(A->done));
-		delete g_amle;
-		g_amle = A = new AmlePlan;
-		A->w = w; A->h = h; A->pd = pd; A->nn = nn; A->niter = niter;
-		A->trace = trace; A->R = R; A->var = var;
 		const size_t n = (size_t)w * h * pd;
-		int rc = A->mem.alloc(&A->c, n);
-		if (!rc && trace) rc = A->mem.alloc(&A->tinf, n);
-		if (!rc && trace) rc = A->mem.alloc(&A->snap, 2 * n);
-		if (!rc) rc = A->mem.alloc(&A->mm, pd);
-		if (!rc) rc = A->mem.alloc((char **)&A->part, spk::amle_part_bytes(w * h, pd));
-		if (!rc && !trace) rc = amle_build(*A, niter);
-		for (int it = 0; !rc && trace && it < niter; it += 10) {
-			rc = amle_build(*A, 1);
-			if (!rc) rc = amle_build(*A, std::min(niter - it - 1, 9));
+		int rc = SP_OK;
+		for (bool stream = true;; stream = false) {
+			delete g_amle;
+			g_amle = A = new AmlePlan;
+			A->mem.stream = stream;
+			A->w = w; A->h = h; A->pd = pd; A->nn = nn; A->niter = niter;
+			A->trace = trace; A->R = R; A->var = var;
+			rc = A->mem.alloc(&A->c, n);
+			if (!rc && trace) rc = A->mem.alloc(&A->tinf, n);
+			if (!rc && trace) rc = A->mem.alloc(&A->snap, 2 * n);
+			if (!rc) rc = A->mem.alloc(&A->mm, pd);
+			if (!rc) rc = A->mem.alloc((char **)&A->part, spk::amle_part_bytes(w * h, pd));
+			if (!rc && !trace) rc = amle_build(*A, niter);
+			for (int it = 0; !rc && trace && it < niter; it += 10) {
+				rc = amle_build(*A, 1);
+				if (!rc) rc = amle_build(*A, std::min(niter - it - 1, 9));
+			}
+			// no room for the streaming sweeps' scratch: in tiles
+			if (rc != SP_ERR_NOMEM || !A->mem.streamed) break;
 		}
 		if (rc) { delete g_amle; g_amle = nullptr; return rc; }
 	}

@@ -222,7 +222,8 @@ int sp_last_cg_trace(int plane, int level, int *n, double *rr, int cap);
  * signature (sizes, buffer addresses, parameters), least recently used
  * first out: at most max_plans plans and max_bytes device bytes (defaults
  * 256 and 16 GiB).  A plan that cannot be allocated empties the cache and
- * is tried once more.  sp_plan_cache_clear frees every cached plan.  No
+ * is tried once more, then without the streaming sweeps' scratch (in tiles:
+ * same results).  sp_plan_cache_clear frees every cached plan.  No
  * reference counterpart. */
 void sp_plan_cache_limit(int max_plans, size_t max_bytes);
 void sp_plan_cache_clear(void);
