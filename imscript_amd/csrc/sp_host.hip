@@ -534,6 +534,8 @@ struct Plan {
 	// where each plane's values after the first sweeps are added up (the
 	// adjoint's sweeps, one level without data terms); empty: not asked for
 	std::vector<float *> acc;
+	float *hist = nullptr;           // room for the values after every sweep
+	size_t hist_floats = 0;          // (the streaming sweeps' summing form)
 	int transpose = 0;               // the CG applies the transposed biharmonic
 	                                 // operator (the adjoint's solve)
 	std::vector<char> key;           // identity of the call this plan serves
@@ -692,6 +694,45 @@ static int gs_build(Plan &pl, LevelPlan &L, int var)
 	return SP_OK;
 }
 
+// form of the streaming sweeps: the default 10 sweeps fill one block of 5
+// wavefronts of 2, whose phases are short (1920 x 1080 x 3: 543 us, by 4 of 4
+// 675, by 4 of 8 1067); where the tasks wait for each other more than for the
+// vector units, the short phases also pay for more blocks of sweeps (AMLE of
+// 1500 x 2500, 80 sweeps: 892 us, by 4 of 4 1035; 1024 x 1024, 100: 513 and
+// 556), else not (512 x 512, 2000: 2.8 ms and 2.2; 4096 x 4096 x 3, 64: 3.2
+// and 2.9)
+static int ss_form_of(int tmax, double px)
+{
+	return tmax <= 20 || (tmax <= 128 && px * tmax < 2e9) ? 1 : 0;
+}
+
+// floats that the values after every sweep of a plane take
+static size_t ss_hist_floats(int form, int w, int h, int T)
+{
+	int K, KT;
+	spk::ss_form_shape(form, K, KT);
+	const int full = (T - 1) / KT * KT;   // whole blocks, then wavefronts of K
+	return (size_t)(full + (T - full + K - 1) / K * K) * (spk::ss_bands(h) + 1)
+		* spk::ss_band_floats(w, KT);
+}
+
+// the planes whose skewed layout a 32-bit byte offset reaches (the summing
+// form's, the values after K sweeps)
+static bool ss_fits(int form, int w, int h, bool sum)
+{
+	int K, KT;
+	spk::ss_form_shape(form, K, KT);
+	return w >= 4 && h >= 4 && 4.0 * (spk::ss_bands(h) + 1) * spk::ss_band_floats(w, KT)
+		< (sum ? 1.0e9 : 4.0e9);
+}
+
+// SIMPOIS_HIP_GS_SHAPE (read when a plan is built) asks for the tiles
+static bool ss_wanted()
+{
+	const char *shape = getenv("SIMPOIS_HIP_GS_SHAPE");
+	return g_gs_flow && !(shape && *shape);
+}
+
 // Whether planes (u, c, w, h, T and t of each set in `in`) can be swept by the
 // streaming kernel, and its data if so, in memory of pl.  It takes positive
 // steps (the coefficient marks a known pixel by a negative zero) and planes
@@ -709,22 +750,13 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bo
 		tmax = std::max(tmax, I.T);
 		px += (double)I.w * I.h;
 	}
-	// the default 10 sweeps fill one block of 5 wavefronts of 2, whose phases
-	// are short (1920 x 1080 x 3: 543 us, by 4 of 4 675, by 4 of 8 1067);
-	// where the tasks wait for each other more than for the vector units, the
-	// short phases also pay for more blocks of sweeps (AMLE of 1500 x 2500, 80
-	// sweeps: 892 us, by 4 of 4 1035; 1024 x 1024, 100: 513 and 556), else not
-	// (512 x 512, 2000: 2.8 ms and 2.2; 4096 x 4096 x 3, 64: 3.2 and 2.9)
-	ss.form = tmax <= 20 || (tmax <= 128 && px * tmax < 2e9) ? 1 : 0;
+	ss.form = ss_form_of(tmax, px);
 	ss.op = op;
 	ss.sum = sum;
 	int K, KT;
 	spk::ss_form_shape(ss.form, K, KT);
-	for (const spk::SsInst &I : in) {
-		if (I.w < 4 || I.h < 4 || !(I.t > 0)) return SP_OK;
-		if (4.0 * (spk::ss_bands(I.h) + 1) * spk::ss_band_floats(I.w, KT) >= (sum ? 1.0e9 : 4.0e9))
-			return SP_OK;
-	}
+	for (const spk::SsInst &I : in)
+		if (!(I.t > 0) || !ss_fits(ss.form, I.w, I.h, sum)) return SP_OK;
 	std::vector<spk::SsBlock> bw;
 	struct Key { int key; spk::SsTask t; };
 	std::vector<Key> tasks;
@@ -744,8 +776,8 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bo
 		const int nT = (T + KT - 1) / KT;
 		if (sum) {
 			I.hs = (nb + 1) * BS;
-			const int last = T - (nT - 1) * KT;   // sweeps of the last block
-			nhist += ((size_t)(nT - 1) * KT + (last + K - 1) / K * K) * I.hs;
+			I.hist = pl.hist + nhist;
+			nhist += ss_hist_floats(ss.form, w, h, T);
 		}
 		prog_off.push_back(nprog);
 		nprog += (size_t)nT * I.nslot * spk::SS_PS;
@@ -760,21 +792,21 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bo
 		for (int jb = 0; jb < (int)nb; jb++)
 			for (int sb = 0; sb * 64 < w + 63; sb++) bw.push_back({(int)id, jb, sb});
 	}
-	if (nprog > 0x7ffffff0 || tasks.size() > 0x7fffffff) return SP_OK;
+	if (nprog > 0x7ffffff0 || tasks.size() > 0x7fffffff || nhist > pl.hist_floats) return SP_OK;
 	std::stable_sort(tasks.begin(), tasks.end(),
 			[](const Key &a, const Key &b) { return a.key < b.key; });
-	// one allocation for all planes (coefficients, values, the values after
-	// every sweep, what bands hand over, progress words with the claim counter
-	// and the level's largest values) and one for the descriptors.  The first
+	// one allocation for all planes (coefficients, values, what bands hand
+	// over, progress words with the claim counter and the level's largest
+	// values) and one for the descriptors.  The first
 	// call on 40 images 100 to 750 pixels wide takes 3.1 ms, with three
 	// allocations and a clearing launch per plane 5.5 (tiles 3.9); dropping
 	// the plans of ten such calls 18 ms instead of 230
 	nbz = rup64(nbz);
 	float *pool = nullptr;
 	pl.streamed = true;
-	TRY(pl.alloc(&pool, 2 * ncell + nbz + nprog + 3 + nhist));
+	TRY(pl.alloc(&pool, 2 * ncell + nbz + nprog + 3));
 	spk::launch_ss_clear(ss.op, pool, ncell, nullptr);
-	float *C = pool, *A = pool + ncell, *hist = pool + 2 * ncell, *const bz = hist + nhist;
+	float *C = pool, *A = pool + ncell, *const bz = pool + 2 * ncell;
 	ss.d_prog = (int *)(bz + nbz);
 	HIPCHK(hipMemset(ss.d_prog, 0, (nprog + 3) * sizeof(int)));
 	ss.d_claim = (unsigned *)ss.d_prog + nprog;
@@ -789,11 +821,6 @@ static int ss_build(Plan &pl, SsRun &ss, std::vector<spk::SsInst> in, int op, bo
 		I.bz = bz + bz_off[k];
 		I.prog = ss.d_prog + prog_off[k];
 		I.mx = ss.d_mx;
-		if (sum) {
-			I.hist = hist;
-			const int nT = (I.T + KT - 1) / KT, last = I.T - (nT - 1) * KT;
-			hist += ((size_t)(nT - 1) * KT + (last + K - 1) / K * K) * I.hs;
-		}
 	}
 	TRY(gs_err_ensure(pl));
 	std::vector<spk::SsTask> tl;
@@ -830,11 +857,10 @@ static void ss_run(Plan &pl, const SsRun &ss, const spk::SsInst *d_inst, hipStre
 	spk::launch_ss_out(d_inst, ss.d_bw, ss.nbw, (unsigned *)ss.d_prog, ss.nprog + 3, s);
 }
 
-// a level's tiled members; SIMPOIS_HIP_GS_SHAPE asks for the tiles
+// a level's tiled members
 static int ss_level(Plan &pl, LevelPlan &L, bool has_f)
 {
-	const char *shape = getenv("SIMPOIS_HIP_GS_SHAPE");
-	if (pl.R != 1 || (shape && *shape)) return SP_OK;
+	if (pl.R != 1 || !ss_wanted()) return SP_OK;
 	std::vector<spk::SsInst> in;
 	for (int m : L.tiled) {
 		spk::SsInst I{};
@@ -2331,6 +2357,102 @@ static int as_err_ensure()
 	return SP_OK;
 }
 
+// Sweeps of one run of the summing forms on level L, and the floats of
+// history that the run takes; 0: neither form takes the level.  By diagonal
+// (no history) as many as its tables allow, by bands as many as AS_HIST floats
+// hold: a layout of narrow planes is many times their pixels (64 x 64: 8, 4
+// columns: over 100).
+constexpr size_t AS_HIST = (size_t)1 << 28;   // 1 GiB, for all levels together
+
+static int as_group(const AsLevel &L, int pd, size_t *floats)
+{
+	*floats = 0;
+	for (int T = L.nsweep;; T -= T / 2) {
+		const int dl = g_gsd_lds > 0 ? spk::gs_diag_lds(L.w, L.h, T, false, true) : 0;
+		if (dl > 0 && dl <= g_gsd_lds) return T;
+		if (T <= 1) break;
+	}
+	for (int T = L.nsweep; ss_wanted(); T -= T / 2) {
+		const int form = ss_form_of(T, (double)L.n * pd);
+		if (!ss_fits(form, L.w, L.h, true)) return 0;
+		const double n = (double)pd * ss_hist_floats(form, L.w, L.h, T);
+		if (n <= (double)AS_HIST) {
+			*floats = (size_t)n;
+			return T;
+		}
+		if (T <= 1) break;
+	}
+	return 0;
+}
+
+// sum: with the summing sweeps where a level can take them, else one sweep at
+// a time in tiles
+static int as_build(AsScratch &A, const std::vector<std::pair<int, int>> &shp, int pd,
+		const sp_params &P, bool sum)
+{
+	A.lv.resize(shp.size());
+	sp_params P1 = P;
+	P1.niter = 1; P1.scale = 1; P1.cgit = 0; P1.ponlit = 0; P1.autotune = 0;
+	P1.guidance = 0; P1.trace = 0;
+	// the levels run one after another and share one history
+	float *hist = nullptr;
+	size_t hist_floats = 0;
+	for (size_t k = 0; k < shp.size(); k++) {
+		AsLevel &L = A.lv[k];
+		L.w = shp[k].first;
+		L.h = shp[k].second;
+		L.n = (size_t)L.w * L.h;
+		// PONLIT: only the level of that width sweeps (simpois.c:271-272)
+		L.nsweep = P.ponlit && P.ponlit != L.w ? 0 : std::max(P.niter, 0);
+		size_t need = 0;
+		if (sum && L.nsweep) L.group = as_group(L, pd, &need);
+		hist_floats = std::max(hist_floats, need);
+	}
+	if (hist_floats) TRY(A.mem.alloc(&hist, hist_floats));
+	for (AsLevel &L : A.lv) {
+		const size_t m = L.n * pd;
+		TRY(A.mem.alloc(&L.hole, m));
+		TRY(A.mem.alloc(&L.v, m));
+		TRY(A.mem.alloc(&L.gg, m));
+		TRY(A.mem.alloc(&L.gf, m));
+		TRY(A.mem.alloc(&L.gi, m));
+		if (!L.nsweep) continue;
+		TRY(A.mem.alloc(&L.g_rot, m));
+		TRY(A.mem.alloc(&L.f_rot, m));
+		TRY(A.mem.alloc(&L.u_rot, m));
+		TRY(A.mem.alloc(&L.acc, m));
+		std::vector<PlaneIn> planes;
+		for (int l = 0; l < pd; l++)
+			planes.push_back(PlaneIn{L.w, L.h, L.g_rot + L.n * l, L.f_rot + L.n * l,
+				L.u_rot + L.n * l});
+		L.sweep = new Plan;
+		L.sweep->gs_err = g_as_err->gs_err;
+		L.sweep->stream = sum;
+		TRY(plan_create(*L.sweep, planes, P1, true));
+		for (PlaneIn &q : planes) q.f = nullptr;
+		for (int part = 0; part < 2 && L.group; part++) {
+			sp_params P2 = P1;
+			P2.niter = part ? L.nsweep % L.group : L.group;
+			if (!P2.niter) break;
+			Plan *pl = new Plan;
+			pl->gs_err = g_as_err->gs_err;
+			(part ? L.rest : L.sum) = pl;
+			for (int l = 0; l < pd; l++) pl->acc.push_back(L.acc + L.n * l);
+			pl->hist = hist;
+			pl->hist_floats = hist_floats;
+			TRY(plan_create(*pl, planes, P2, false));
+			// planes that the summing forms do not take
+			if (!pl->lv[0].tiled.empty() && !pl->lv[0].ss.nt) {
+				delete L.sum;
+				delete L.rest;
+				L.sum = L.rest = nullptr;
+				L.group = 0;
+			}
+		}
+	}
+	return SP_OK;
+}
+
 static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 {
 	std::vector<std::pair<int, int>> shp;
@@ -2346,67 +2468,20 @@ static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 	memcpy(&step, &P.tstep, sizeof step);
 	std::vector<int> key = {w, h, pd, (int)shp.size(), P.niter, (int)P.ponlit, step};
 	if (g_as && g_as->key == key) { *out = g_as; return SP_OK; }
-	delete g_as;
-	g_as = nullptr;
-	AsScratch *A = new AsScratch;
-	A->key = key;
-	A->lv.resize(shp.size());
-	sp_params P1 = P;
-	P1.niter = 1; P1.scale = 1; P1.cgit = 0; P1.ponlit = 0; P1.autotune = 0;
-	P1.guidance = 0; P1.trace = 0;
-	int rc = SP_OK;
-	for (size_t k = 0; k < shp.size() && !rc; k++) {
-		AsLevel &L = A->lv[k];
-		L.w = shp[k].first;
-		L.h = shp[k].second;
-		L.n = (size_t)L.w * L.h;
-		// PONLIT: only the level of that width sweeps (simpois.c:271-272)
-		L.nsweep = P.ponlit && P.ponlit != L.w ? 0 : std::max(P.niter, 0);
-		const size_t m = L.n * pd;
-		rc = A->mem.alloc(&L.hole, m);
-		if (!rc) rc = A->mem.alloc(&L.v, m);
-		if (!rc) rc = A->mem.alloc(&L.gg, m);
-		if (!rc) rc = A->mem.alloc(&L.gf, m);
-		if (!rc) rc = A->mem.alloc(&L.gi, m);
-		if (rc || !L.nsweep) continue;
-		rc = A->mem.alloc(&L.g_rot, m);
-		if (!rc) rc = A->mem.alloc(&L.f_rot, m);
-		if (!rc) rc = A->mem.alloc(&L.u_rot, m);
-		if (!rc) rc = A->mem.alloc(&L.acc, m);
-		if (rc) break;
-		std::vector<PlaneIn> planes;
-		for (int l = 0; l < pd; l++)
-			planes.push_back(PlaneIn{L.w, L.h, L.g_rot + L.n * l, L.f_rot + L.n * l,
-				L.u_rot + L.n * l});
-		L.sweep = new Plan;
-		L.sweep->gs_err = g_as_err->gs_err;
-		rc = plan_create(*L.sweep, planes, P1, true);
-		if (rc) break;
-		// the summing sweeps hold the values after each of them: at most
-		// 1 GiB per call
-		L.group = (int)std::min<double>(L.nsweep, std::max(1.0, 2.4e8 / (1.2 * m)));
-		for (PlaneIn &q : planes) q.f = nullptr;
-		for (int part = 0; part < 2 && !rc; part++) {
-			sp_params P2 = P1;
-			P2.niter = part ? L.nsweep % L.group : L.group;
-			if (!P2.niter) break;
-			Plan *pl = new Plan;
-			pl->gs_err = g_as_err->gs_err;
-			(part ? L.rest : L.sum) = pl;
-			for (int l = 0; l < pd; l++) pl->acc.push_back(L.acc + L.n * l);
-			rc = plan_create(*pl, planes, P2, false);
-			// planes that the summing forms do not take
-			if (!rc && !pl->lv[0].tiled.empty() && !pl->lv[0].ss.nt) {
-				delete L.sum;
-				delete L.rest;
-				L.sum = L.rest = nullptr;
-				break;
-			}
+	// where the summing sweeps do not fit: one sweep at a time, in tiles
+	for (const bool sum : {true, false}) {
+		delete g_as;
+		g_as = nullptr;
+		AsScratch *A = new AsScratch;
+		A->key = key;
+		const int rc = as_build(*A, shp, pd, P, sum);
+		if (rc == SP_OK) {
+			*out = g_as = A;
+			return SP_OK;
 		}
+		delete A;
+		if (rc != SP_ERR_NOMEM || !sum) return rc;
 	}
-	if (rc) { delete A; return rc; }
-	g_as = A;
-	*out = A;
 	return SP_OK;
 }
 
