@@ -2716,6 +2716,7 @@ struct AmleSched {
 
 struct AmlePlan {
 	int w = 0, h = 0, pd = 0, nn = 0, niter = 0, trace = 0, R = 1, var = 0;
+	bool stream = false;              // streaming sweeps wanted (else tiles)
 	Plan mem;                         // owns the device buffers
 	float *c = nullptr, *tinf = nullptr, *snap = nullptr;
 	float2 *mm = nullptr;
@@ -2744,9 +2745,8 @@ static int amle_build(AmlePlan &A, int T)
 	std::vector<GsTile> tiles;
 	AmleSched sc;
 	sc.T = T;
-	// the streaming sweeps, unless a tile shape is asked for; the output
-	// buffer's planes are bound by amle_bind
-	if (A.nn == 4 && !getenv("SIMPOIS_HIP_AMLE_VARIANT")) {
+	// (the output buffer's planes are bound by amle_bind)
+	if (A.stream) {
 		std::vector<spk::SsInst> in;
 		for (int l = 0; l < ninst; l++) {
 			spk::SsInst I{};
@@ -2894,14 +2894,18 @@ static AmlePlan *g_amle = nullptr;
 static int amle_run(AmlePlan &A, float *d_out, const float *d_in, const float *d_init,
 		hipStream_t s);
 
-// tile shape of the 4-neighbour sweeps: SIMPOIS_HIP_AMLE_VARIANT (read at
-// each call), else 32x32x16 (variant 6) for one plane, whose wavefronts hold
-// few tiles, and 32x64x16 (variant 0) for several (measured on 4096^2
-// planes); variant 0 for the larger neighbourhoods
-static int amle_variant(int R, int pd)
+// how the sweeps run: SIMPOIS_HIP_AMLE_VARIANT (read at each call; empty: not
+// set) asks for the tiles, in that shape for 4 neighbours.  Without it 4
+// neighbours stream, and tiles where the bands do not apply are 32x32x16
+// (variant 6) for one plane, whose wavefronts hold few tiles, and 32x64x16
+// (variant 0) for several (measured on 4096^2 planes); variant 0 for the
+// larger neighbourhoods.
+static int amle_variant(int R, int nn, int pd, bool *stream)
 {
 	const char *e = getenv("SIMPOIS_HIP_AMLE_VARIANT");
-	const int v = e ? atoi(e) : pd == 1 ? 6 : 0;
+	const bool asked = e && *e;
+	const int v = asked ? atoi(e) : pd == 1 ? 6 : 0;
+	*stream = nn == 4 && !asked;
 	return R == 1 && v > 0 && v < amle_shape_count(1) ? v : 0;
 }
 
@@ -2913,7 +2917,8 @@ extern "C" int sp_amle_device(float *d_out, const float *d_in, const float *d_in
 	hipStream_t s = (hipStream_t)stream;
 	std::lock_guard<std::mutex> lk(g_amle_mu);
 	const int R = amle_radius(nn);
-	const int var = amle_variant(R, pd);
+	bool streams;
+	const int var = amle_variant(R, nn, pd, &streams);
 	trace = trace != 0;
 	AmlePlan *A = g_amle;
 	// a dependence wait of an earlier call that timed out (the calls are
@@ -2925,7 +2930,7 @@ extern "C" int sp_amle_device(float *d_out, const float *d_in, const float *d_in
 		return set_err(SP_ERR_HIP, "AMLE tile dependence wait timed out in an earlier call");
 	}
 	if (!A || A->w != w || A->h != h || A->pd != pd || A->nn != nn ||
-			A->niter != niter || A->trace != trace || A->var != var) {
+			A->niter != niter || A->trace != trace || A->var != var || A->stream != streams) {
 		// the old plan's scratch may still be in use on its stream
 		if (A && A->used) HIPCHK(hipEventSynchronize(A->done));
 		const size_t n = (size_t)w * h * pd;
@@ -2935,7 +2940,7 @@ extern "C" int sp_amle_device(float *d_out, const float *d_in, const float *d_in
 			g_amle = A = new AmlePlan;
 			A->mem.stream = stream;
 			A->w = w; A->h = h; A->pd = pd; A->nn = nn; A->niter = niter;
-			A->trace = trace; A->R = R; A->var = var;
+			A->trace = trace; A->R = R; A->var = var; A->stream = streams;
 			rc = A->mem.alloc(&A->c, n);
 			if (!rc && trace) rc = A->mem.alloc(&A->tinf, n);
 			if (!rc && trace) rc = A->mem.alloc(&A->snap, 2 * n);
