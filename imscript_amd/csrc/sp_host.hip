@@ -876,23 +876,27 @@ static int ss_level(Plan &pl, LevelPlan &L, bool has_f)
 //
 // With sp_params.autotune set, the first sweep of a level whose members run
 // in tiles times every compiled tile shape of its radius (sp_gs.h) on a
-// scratch copy of the level's current data, keeps the fastest, and caches
-// the choice for the process under (radius, sweeps, member sizes).  Every
-// shape runs the same lexicographic schedule, so the choice never changes
-// the result, only the time.
+// scratch copy of the level's current data, and the streaming sweeps where
+// the level can take them, keeps the fastest, and caches the choice for the
+// process (gs_key).  Every one runs the same lexicographic schedule, so the
+// choice never changes the result, only the time.
 
 struct TuneRec {
 	std::vector<long> key;
 	int var;
 	std::vector<float> ms;   // per variant
-	float ss_ms;             // streaming sweeps (1e30: the level cannot take them)
+	float ss_ms;             // streaming sweeps (1e30: not available to it)
 };
 static std::mutex g_tune_mu;
 static std::vector<TuneRec> g_tune;
 
+// what a choice depends on: the radius, the streaming sweeps' code (0: not
+// available; else their operator, and whether small values are certain, which
+// leaves out the finite tests) and the sizes and sweeps of the members
+static constexpr size_t GS_KEY_HEAD = 2;
 static std::vector<long> gs_key(const Plan &pl, const LevelPlan &L)
 {
-	std::vector<long> k = {pl.R};
+	std::vector<long> k = {pl.R, L.ss.nt ? 1 + 2 * L.ss.op + L.ss.small : 0};
 	for (int m : L.tiled) {
 		k.push_back(L.sp[m].w);
 		k.push_back(L.sp[m].h);
@@ -1027,9 +1031,10 @@ extern "C" int sp_autotune_report(char *buf, int cap)
 		const int R = (int)r.key[0];
 		char line[256];
 		long px = 0;
-		for (size_t z = 1; z + 2 < r.key.size(); z += 3) px += r.key[z] * r.key[z + 1];
+		const size_t h0 = GS_KEY_HEAD;
+		for (size_t z = h0; z + 2 < r.key.size(); z += 3) px += r.key[z] * r.key[z + 1];
 		snprintf(line, sizeof line, "gs R=%d T=%ld planes=%d px=%ld choice=", R,
-				r.key.size() > 3 ? r.key[3] : 0L, (int)(r.key.size() - 1) / 3, px);
+				r.key.size() > h0 + 2 ? r.key[h0 + 2] : 0L, (int)((r.key.size() - h0) / 3), px);
 		out += line;
 		for (int v = 0; v < (int)r.ms.size(); v++) {
 			sp_with_shape(R, v, [&](auto sh) {
