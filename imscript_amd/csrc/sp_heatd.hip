@@ -122,9 +122,11 @@ __global__ __launch_bounds__(HD_T) void k_heatd_step(float *__restrict__ out,
 // overflows; the host's choice) takes a short form: no corner can matter, the
 // leading 0 + N and the exact product -4 C fold into the additions, and the
 // west and east neighbours are operands of theirs (lane shifts): 7 vector
-// operations per cell instead of 14 and two LDS permutes.  4096 x 4096 x 3,
-// 100 steps: 2.1 ms instead of 3.4 (125 us per launch of 6 steps, 79 of them
-// the time a copy of the planes takes).
+// operations per cell instead of 14.  4096 x 4096 x 3, 100 steps: 2.1 ms
+// instead of 3.4 (125 us per launch of 6 steps, 79 of them the time a copy of
+// the planes takes).  The general form takes its neighbours by lane shifts
+// too: where all tiles are of it, 1024 x 1024, 60 steps 218 us (by LDS
+// permutes 281, and 255 without the short form beside it).
 
 constexpr int HT_R = 48;          // rows per wave tile
 constexpr int HT_WAVES = 4;       // wave tiles per block, stacked vertically
@@ -226,7 +228,7 @@ void k_heatd_multi(float *__restrict__ out,
 		// the corners of row r are the west / east neighbours of rows r-1
 		// and r+1: whether a row's pair is finite is kept with the row
 		float c = v[0];
-		float cw = __shfl_up(c, 1, 64), ce = __shfl_down(c, 1, 64);
+		float cw = hd_west(c), ce = hd_east(c);
 		if (edge_cols) { cw = atl ? c : cw; ce = atr ? c : ce; }
 		bool cf = isfinite(cw) && isfinite(ce);
 		float u = c;
@@ -234,7 +236,7 @@ void k_heatd_multi(float *__restrict__ out,
 #pragma unroll
 		for (int r = 0; r < HT_R; r++) {
 			const float d = r + 1 < HT_R ? v[r + 1] : c;
-			float dw = __shfl_up(d, 1, 64), de = __shfl_down(d, 1, 64);
+			float dw = hd_west(d), de = hd_east(d);
 			if (edge_cols) { dw = atl ? d : dw; de = atr ? d : de; }
 			const bool df = isfinite(dw) && isfinite(de);
 			float n = u, so = d;
