@@ -2743,6 +2743,22 @@ static AmleSched *amle_sched(AmlePlan &A, int T)
 	return nullptr;
 }
 
+// Whether T sweeps of a plane are so few tiles that their one launch takes
+// less than the bands' three: two wavefronts of tiles, or three where the
+// tiles hold little.  us, tiles / bands: 16 x 16, 10 sweeps 44 / 70; 24 x 24,
+// 16 sweeps 68 / 75; 32 x 32, 5 sweeps 67 / 70, 10 sweeps 71 / 70; 64 x 64, 1
+// sweep 74 / 78, 5 sweeps (5 wavefronts) 103 / 84; 56 x 56, 5 sweeps 78 / 70;
+// 16 x 16, 20 sweeps (two passes) 76 / 78.
+static bool amle_few_tiles(const AmlePlan &A, int T)
+{
+	int nI = 0, nJ = 0, nT = 0;
+	amle_with_shape(A.R, A.var, [&](auto sh) {
+		tile_grid<decltype(sh)>(A.w, A.h, T, nI, nJ, nT);
+	});
+	return nT == 1 && (nI + nJ <= 3
+			|| (nI + nJ == 4 && (T <= 2 || std::max(A.w, A.h) <= 32)));
+}
+
 static int amle_build(AmlePlan &A, int T)
 {
 	if (T <= 0 || amle_sched(A, T)) return SP_OK;
@@ -2751,7 +2767,7 @@ static int amle_build(AmlePlan &A, int T)
 	AmleSched sc;
 	sc.T = T;
 	// (the output buffer's planes are bound by amle_bind)
-	if (A.stream) {
+	if (A.stream && !amle_few_tiles(A, T)) {
 		std::vector<spk::SsInst> in;
 		for (int l = 0; l < ninst; l++) {
 			spk::SsInst I{};
