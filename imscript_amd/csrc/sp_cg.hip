@@ -336,14 +336,13 @@ __global__ __launch_bounds__(NT) void k32_setup(const BlockWork *bw,
 		// right-hand side), x only in groups with an unknown.  The
 		// biharmonic iteration starts from p = r, and its product reads p
 		// at every pixel of the 13-point stencil, unknown or not: p and q
-		// everywhere, and z, of which p takes whole groups.  (The Poisson
-		// iteration writes p and q itself.)
+		// everywhere (its z is r: no multigrid).  (The Poisson iteration
+		// writes p and q itself.)
 		gstore<unsigned>(P.code + q4, cc);
 		gstore<f4>(P.r + q4, rv);
 		if (P.bilap) {
 			gstore<f4>(P.p + q4, rv);
 			gstore<f4>(P.q + q4, f4{0.0f, 0.0f, 0.0f, 0.0f});
-			if (P.z != P.r) gstore<f4>(P.z + q4, f4{0.0f, 0.0f, 0.0f, 0.0f});
 		}
 		if (cc & 0x01010101u) gstore<d4>(P.x + q4, xv);
 	}
