@@ -2,7 +2,8 @@
 #pragma once
 #include "sp_internal.h"
 
-// one plane of the batched CG: full-grid float vectors, zero at known pixels
+// one plane of the batched CG: full-grid float vectors (at known pixels: see
+// the vector kernels, sp_cg.hip)
 struct Cg32Plane {
 	const float *g;    // boundary data, NaN = unknown
 	const float *f;    // data term or nullptr

@@ -27,8 +27,11 @@ static_assert(NT * PPT == 1024, "work blocks span 1024 pixels");
 
 // Vector kernels below give each thread the 4 consecutive pixels
 // start + 4 tid .. + 3 of its work block (plane vectors start 256-byte
-// aligned).  Known pixels hold x = r = p = q = z = 0 throughout, so a group
-// with at least one unknown is updated whole: the known entries stay 0.
+// aligned).  In a group with at least one unknown the known pixels hold x =
+// r = p = q = 0 throughout, so such a group is updated whole: its known entries
+// stay 0.  z is r without multigrid.  With it, known pixels may hold anything
+// in z (the level-0 strips write no pair of known pixels): only k32_dirspmv
+// reads it, and takes every value under the code bits.
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 
@@ -2348,8 +2351,8 @@ static void vcycle(const Cg32Batch &B, hipStream_t s)
 	});
 	if (B.prof) B.prof("mg_down0", 0, 10.0 * B.px0, s);
 	// levels >= 1 outside the tail: fused tiles (packed coefficients; per
-	// cell down reads b and the code, writes zd and a quarter coarse b and
-	// z, 14 B; up reads zd, b, the code and a quarter coarse z, writes z,
+	// cell down reads b and the code, writes zd and a quarter coarse b, 13 B;
+	// up reads zd, b, the code and a quarter coarse z, writes z,
 	// 17 B; 4 B more per cell for the two-word codes) or per-level kernels
 	// (pre-smooth, restrict)
 	for (int l = 1; l < L; l++) {
@@ -2368,7 +2371,7 @@ static void vcycle(const Cg32Batch &B, hipStream_t s)
 			else
 				with_geo<GeoC, MG_NGEO>(W.geo, [&](auto g) { down(LevG64{}, g); });
 			if (B.prof)
-				B.prof(g_down_name[l], 0, (l > MG_G32_MAX ? 18.0 : 14.0) * W.cells, s);
+				B.prof(g_down_name[l], 0, (l > MG_G32_MAX ? 17.0 : 13.0) * W.cells, s);
 		}
 		if (!W.nmid) continue;
 		for (int it = 0; it < B.nu; it++) {

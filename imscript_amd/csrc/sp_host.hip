@@ -694,13 +694,18 @@ static int gs_build(Plan &pl, LevelPlan &L, int var)
 	return SP_OK;
 }
 
-// form of the streaming sweeps: the default 10 sweeps fill one block of 5
-// wavefronts of 2, whose phases are short (1920 x 1080 x 3: 543 us, by 4 of 4
-// 675, by 4 of 8 1067); where the tasks wait for each other more than for the
-// vector units, the short phases also pay for more blocks of sweeps (AMLE of
-// 1500 x 2500, 80 sweeps: 892 us, by 4 of 4 1035; 1024 x 1024, 100: 513 and
-// 556), else not (512 x 512, 2000: 2.8 ms and 2.2; 4096 x 4096 x 3, 64: 3.2
-// and 2.9)
+// form of the streaming sweeps: 2 sweeps a wavefront (1) or 4 (0).  The default
+// 10 sweeps fill one block of 5 wavefronts of 2, whose phases are short (1920 x
+// 1080 x 3: 543 us, by 4 of 4 675, by 4 of 8 1067).  Where the tasks wait for
+// each other more than for the vector units, the short phases also pay for
+// more blocks of sweeps.  A level of that many sweeps, us, by 2 / by 4:
+//   512 x 512       64: 342 / 358   100: 396 / 401   128: 427 / 422   200: 533 / 507
+//   1024 x 1024     64: 538 / 583   128: 628 / 654   160: 681 / 694   200: 751 / 742
+//   1920 x 1080 x 3 64: 771 / 819   128: 985 / 984   160: 1094 / 1049
+//   2048 x 2048 x 3 64: 1173 / 1263   100 (1.3e9 updates): 1354 / 1360   128: 1504 / 1446
+//   4096 x 4096 x 3 32 (1.6e9): 2687 / 2839   48 (2.4e9): 3010 / 2996   64: 3455 / 3132
+// so both lines lie where the forms break even.  (200 x 200 would break even at
+// 48 sweeps, 208 / 208; 128: 320 / 296.)
 static int ss_form_of(int tmax, double px)
 {
 	return tmax <= 20 || (tmax <= 128 && px * tmax < 2e9) ? 1 : 0;
@@ -1185,7 +1190,14 @@ static int plan_create(Plan &pl, const std::vector<PlaneIn> &planes,
 				const int w = L.sp[m].w, h = L.sp[m].h, T = L.nsweep[m];
 				if (T <= 0) continue;
 				// few sweeps against the level's diagonals: by diagonal (the
-				// form that sums has no other)
+				// form that sums has no other).  A call on one such level, us,
+				// by diagonal / by cells, 40 % holes: 128 x 128, 32 sweeps 161 /
+				// 250, 64 (the line) 222 / 305, 128: 351 / 423, 320: 731 / 778;
+				// 16 x 900, 229 (the line) 626 / 901, 687: 1433 / 1852; 64 x 64,
+				// 32 (the line) 93 / 103, 160: 194 / 201, with 90 % holes 251 /
+				// 240; 32 x 32, 16 (the line) 57 / 58, 80: 96 / 91.  The line is
+				// where the smallest levels stop gaining; larger ones gain
+				// beyond it too.
 				const int dl = g_gsd_lds > 0 ? spk::gs_diag_lds(w, h, T, has_f, sum) : 0;
 				if (dl > 0 && dl <= g_gsd_lds && (sum || 4 * T <= w + h)) {
 					diag.push_back(m);
