@@ -2768,12 +2768,12 @@ static AmleSched *amle_sched(AmlePlan &A, int T)
 	return nullptr;
 }
 
-// Whether T sweeps of a plane are so few tiles that their one launch takes
-// less than the bands' three: two wavefronts of tiles, or three where the
-// tiles hold little.  us, tiles / bands: 16 x 16, 10 sweeps 44 / 70; 24 x 24,
-// 16 sweeps 68 / 75; 32 x 32, 5 sweeps 67 / 70, 10 sweeps 71 / 70; 64 x 64, 1
-// sweep 74 / 78, 5 sweeps (5 wavefronts) 103 / 84; 56 x 56, 5 sweeps 78 / 70;
-// 16 x 16, 20 sweeps (two passes) 76 / 78.
+// Whether T sweeps of a plane are so few tiles that a launch per wavefront of
+// them takes less than the bands' three: two wavefronts, or three where the
+// tiles hold little.  us, tiles / bands: 16 x 16, 10 sweeps 38 / 70; 24 x 24, 16
+// sweeps 63 / 76; 32 x 32, 10 sweeps 65 / 72; 64 x 64, 1 sweep 71 / 81; 64 x 64,
+// 5 sweeps (5 wavefronts, in one launch by dependences) 103 / 84; 56 x 56, 5
+// sweeps 74 / 70; 16 x 16, 20 sweeps (two passes) 76 / 78.
 static bool amle_few_tiles(const AmlePlan &A, int T)
 {
 	int nI = 0, nJ = 0, nT = 0;
@@ -2792,7 +2792,8 @@ static int amle_build(AmlePlan &A, int T)
 	AmleSched sc;
 	sc.T = T;
 	// (the output buffer's planes are bound by amle_bind)
-	if (A.stream && !amle_few_tiles(A, T)) {
+	const bool few = A.stream && amle_few_tiles(A, T);
+	if (A.stream && !few) {
 		std::vector<spk::SsInst> in;
 		for (int l = 0; l < ninst; l++) {
 			spk::SsInst I{};
@@ -2818,7 +2819,7 @@ static int amle_build(AmlePlan &A, int T)
 	TRY(A.mem.upload(&sc.d_tiles, tiles));
 	TRY(A.mem.alloc(&sc.d_insts, ninst));
 	sc.ntiles = (int)tiles.size();
-	if (g_gs_flow && !tiles.empty()) {
+	if (g_gs_flow && !tiles.empty() && !few) {
 		// every instance has the same tile grid (flags as in gs_flow_build)
 		GsFlowInst g{0, 0, 0, 0};
 		amle_with_shape(A.R, A.var, [&](auto sh) {

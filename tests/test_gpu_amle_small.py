@@ -1,6 +1,6 @@
-"""GPU: 4-neighbour AMLE of the smallest planes runs in tiles (one launch),
-larger ones stream (three), with the oracle's bits on both sides of the rule,
-zeros of both signs included."""
+"""GPU: 4-neighbour AMLE of the smallest planes runs in tiles (a launch per
+wavefront of them, at most three), larger ones stream (three launches), with
+the oracle's bits on both sides of the rule, zeros of both signs included."""
 import numpy as np
 import pytest
 
@@ -10,9 +10,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("pd,h,w,n,launches", [
-    (1, 16, 16, 16, 1), (1, 16, 16, 17, 3), (1, 32, 32, 16, 1), (1, 33, 32, 16, 3),
-    (1, 63, 63, 2, 1), (1, 64, 64, 2, 3), (1, 62, 62, 3, 3), (1, 16, 62, 3, 1),
-    (3, 90, 12, 16, 1), (3, 33, 65, 16, 3), (2, 4, 4, 1, 1)])
+    (1, 16, 16, 16, 1), (1, 16, 16, 17, 3), (1, 32, 32, 16, 3), (1, 33, 32, 16, 3),
+    (1, 63, 63, 2, 3), (1, 64, 64, 2, 3), (1, 62, 62, 3, 3), (1, 16, 62, 3, 2),
+    (3, 90, 12, 16, 2), (3, 33, 65, 16, 3), (2, 4, 4, 1, 1)])
 def test_both_sides_of_the_rule(pd, h, w, n, launches):
     import torch
     import imscript_amd as m
