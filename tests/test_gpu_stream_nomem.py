@@ -69,22 +69,23 @@ def test_amle_runs_in_tiles(cap, monkeypatch):
     x, _ = _image(1, 500, 620)
     small = torch.full((1, 8, 8), 3.0, device="cuda")
 
-    def amle(n, capped=0):
-        m.amle(small, 4, 1)      # (one plan is kept: the small one)
+    def amle(n, capped=0, variant=None):
+        m.amle(small, 4, 1)      # (one plan is kept: the small one, always alike)
         base = m.device_bytes()
         cap(capped)
+        if variant:
+            monkeypatch.setenv("SIMPOIS_HIP_AMLE_VARIANT", variant)
         try:
             out = m.amle(x, 4, n)
             torch.cuda.synchronize()
         finally:
             cap(0)
+            monkeypatch.delenv("SIMPOIS_HIP_AMLE_VARIANT", raising=False)
         return out, m.device_bytes() - base
 
     print("no room, amle", flush=True)
     want, streamed = amle(30)
-    monkeypatch.setenv("SIMPOIS_HIP_AMLE_VARIANT", "6")
-    _, tiles = amle(30)
-    monkeypatch.delenv("SIMPOIS_HIP_AMLE_VARIANT")
+    _, tiles = amle(30, variant="6")
     assert tiles < streamed
     got, held = amle(30, tiles)
     assert held <= tiles
