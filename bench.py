@@ -44,11 +44,11 @@ PEAK_HBM_GBPS = 8000.0
 # measured on: TRAFFIC_SRC is the SHA-256 prefix of imscript_amd/csrc/sp_cg.hip
 # then, and the line reports traffic null when the source differs.
 TRAFFIC_PMC = {
-    "mg_up0": 554.9e6,
-    "mg_down0": 362.4e6,
-    "k32_dirspmv": 703.2e6,
+    "mg_up0": 553.6e6,
+    "mg_down0": 361.6e6,
+    "k32_dirspmv": 703.3e6,
 }
-TRAFFIC_SRC = "a4df540fb588e47d"
+TRAFFIC_SRC = "4ee8216a8685ca90"
 
 
 def kernel_source_id(name="sp_cg.hip"):

@@ -114,10 +114,11 @@ typedef struct sp_params {
 	int cg_chunk;    /* CG iterations per captured graph (FP32 CG) */
 	int cg_mg;       /* 1: precondition the FP32 CG with a multigrid V-cycle
 	                    (Poisson only); 0: plain CG as the reference */
-	int autotune;    /* 1: time every compiled Gauss-Seidel tile shape on the
-	                    first sweep of each level size and keep the fastest
-	                    (cached per process; results do not depend on it);
-	                    0: built-in shapes.  Default from SIMPOIS_HIP_AUTOTUNE */
+	int autotune;    /* 1: time every compiled Gauss-Seidel tile shape, and the
+	                    streaming bands where they apply, on the first sweep
+	                    of each level size and keep the fastest (cached per
+	                    process; results do not depend on it); 0: bands, or
+	                    built-in shapes.  Default from SIMPOIS_HIP_AUTOTUNE */
 	int guidance;    /* 0: f is the data term, as in the reference; 1 or 2: f
 	                    holds a source image v and the data term is plambda's
 	                    "x,l" (1) or "x,lr" (2) Laplacian of v with the
@@ -340,8 +341,9 @@ int sp_stream_copy(float *d_dst, const float *d_src, size_t n, void *stream);
 
 /* Choices of the tile-shape autotuner so far in this process, one text
  * line per tuned level size: "gs R=<radius> T=<sweeps> planes=<n>
- * px=<pixels> choice=<BIxBJxBT:ms>,..." with the chosen shape prefixed '*'.
- * Writes at most cap bytes (NUL-terminated) and returns the size needed.
+ * px=<pixels> choice=<BIxBJxBT:ms>,...,stream:<ms>" with the choice
+ * prefixed '*' (stream: the streaming bands, where they were timed; calls
+ * whose bands run other code have lines of their own).  Writes at most cap bytes (NUL-terminated) and returns the size needed.
  * No reference counterpart. */
 int sp_autotune_report(char *buf, int cap);
 
