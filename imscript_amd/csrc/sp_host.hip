@@ -2362,8 +2362,9 @@ struct AsLevel {
 };
 
 struct AsScratch {
-	std::vector<int> key;       // w, h, pd, levels, niter, PONLIT
-	Plan mem;                   // owns the level buffers
+	std::vector<int> key;       // w, h, pd, levels, niter, PONLIT, tstep
+	Plan mem;                   // owns the level buffers and the error word of
+	                            // every sweep's dependence waits
 	std::vector<AsLevel> lv;
 	~AsScratch()
 	{
@@ -2372,21 +2373,7 @@ struct AsScratch {
 };
 static std::mutex g_as_mu;
 static AsScratch *g_as = nullptr;
-// error word of the dependence waits of every sweep of a gradient (gs_err /
-// h_gs_err of this object, which lives as long as the process): the images of
-// one call may each replace the scratch, and the call reads the word once
-static Plan *g_as_err = nullptr;
-
-static int as_err_ensure()
-{
-	if (g_as_err) return SP_OK;
-	Plan *E = new Plan;
-	int rc = gs_err_ensure(*E);
-	if (rc) { delete E; return rc; }
-	g_as_err = E;
-	return SP_OK;
-}
-
+static int *g_as_word = nullptr;   // pinned: host copy of a scratch's error word
 // Sweeps of one run of the summing forms on level L, and the floats of
 // history that the run takes; 0: neither form takes the level.  By diagonal
 // (no history) as many as its tables allow, by bands as many as AS_HIST floats
@@ -2421,6 +2408,8 @@ static int as_build(AsScratch &A, const std::vector<std::pair<int, int>> &shp, i
 		const sp_params &P, bool sum)
 {
 	A.lv.resize(shp.size());
+	TRY(A.mem.alloc(&A.mem.gs_err, 1));
+	HIPCHK(hipMemset(A.mem.gs_err, 0, sizeof(int)));
 	sp_params P1 = P;
 	P1.niter = 1; P1.scale = 1; P1.cgit = 0; P1.ponlit = 0; P1.autotune = 0;
 	P1.guidance = 0; P1.trace = 0;
@@ -2456,7 +2445,7 @@ static int as_build(AsScratch &A, const std::vector<std::pair<int, int>> &shp, i
 			planes.push_back(PlaneIn{L.w, L.h, L.g_rot + L.n * l, L.f_rot + L.n * l,
 				L.u_rot + L.n * l});
 		L.sweep = new Plan;
-		L.sweep->gs_err = g_as_err->gs_err;
+		L.sweep->gs_err = A.mem.gs_err;
 		L.sweep->stream = sum;
 		TRY(plan_create(*L.sweep, planes, P1, true));
 		for (PlaneIn &q : planes) q.f = nullptr;
@@ -2465,7 +2454,7 @@ static int as_build(AsScratch &A, const std::vector<std::pair<int, int>> &shp, i
 			P2.niter = part ? L.nsweep % L.group : L.group;
 			if (!P2.niter) break;
 			Plan *pl = new Plan;
-			pl->gs_err = g_as_err->gs_err;
+			pl->gs_err = A.mem.gs_err;
 			(part ? L.rest : L.sum) = pl;
 			for (int l = 0; l < pd; l++) pl->acc.push_back(L.acc + L.n * l);
 			pl->hist = hist;
@@ -2483,7 +2472,24 @@ static int as_build(AsScratch &A, const std::vector<std::pair<int, int>> &shp, i
 	return SP_OK;
 }
 
-static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
+// whether a dependence wait of the scratch's sweeps gave up; the word is
+// cleared.  Waits for the stream's work.
+static bool as_timed_out(AsScratch &A, hipStream_t s)
+{
+	int e = 0;
+	if (hipMemcpyAsync(g_as_word ? g_as_word : &e, A.mem.gs_err, sizeof(int),
+				hipMemcpyDeviceToHost, s) != hipSuccess
+			|| hipStreamSynchronize(s) != hipSuccess)
+		return false;   // (a failed stream is reported by the caller's own checks)
+	if (!(g_as_word ? *g_as_word : e)) return false;
+	(void)hipMemset(A.mem.gs_err, 0, sizeof(int));
+	return true;
+}
+
+// the scratch of one image's shape; timed_out: set where the scratch that it
+// replaces, of an image before in the same call, holds a wait that gave up
+static int as_scratch(int w, int h, int pd, const sp_params &P, hipStream_t s,
+		bool *timed_out, AsScratch **out)
 {
 	std::vector<std::pair<int, int>> shp;
 	for (int cw = w, ch = h, sc = P.scale;;) {
@@ -2498,6 +2504,7 @@ static int as_scratch(int w, int h, int pd, const sp_params &P, AsScratch **out)
 	memcpy(&step, &P.tstep, sizeof step);
 	std::vector<int> key = {w, h, pd, (int)shp.size(), P.niter, (int)P.ponlit, step};
 	if (g_as && g_as->key == key) { *out = g_as; return SP_OK; }
+	if (g_as) *timed_out |= as_timed_out(*g_as, s);
 	// where the summing sweeps do not fit: one sweep at a time, in tiles
 	for (const bool sum : {true, false}) {
 		delete g_as;
@@ -2528,10 +2535,10 @@ static int as_sweep(AsLevel &L, bool prepare, bool start, hipStream_t s)
 
 // the pd planes of one image
 static int adjoint_sweeps_image(const sp_adjoint_image &I, const sp_params &P,
-		hipStream_t s, int *levels)
+		hipStream_t s, int *levels, bool *timed_out)
 {
 	AsScratch *A = nullptr;
-	TRY(as_scratch(I.w, I.h, I.pd, P, &A));
+	TRY(as_scratch(I.w, I.h, I.pd, P, s, timed_out, &A));
 	const int nl = (int)A->lv.size(), np = I.pd;
 	const float t = P.tstep;
 	*levels = std::max(*levels, nl);
@@ -2599,29 +2606,29 @@ static int adjoint_sweeps(int n, const sp_adjoint_image *imgs, const sp_params &
 		return set_err(SP_ERR_ARG, "the adjoint takes the data term itself "
 				"(guidance = 0); differentiate plambda's Laplacian separately");
 	std::lock_guard<std::mutex> lk(g_as_mu);
-	TRY(as_err_ensure());
+	if (!g_as_word && hipHostMalloc((void **)&g_as_word, sizeof(int), hipHostMallocPortable)
+			!= hipSuccess) {
+		(void)hipGetLastError();   // a pageable one then
+		g_as_word = nullptr;
+	}
 	hipEvent_t e0, e1;
 	HIPCHK(hipEventCreate(&e0));
 	HIPCHK(hipEventCreate(&e1));
 	HIPCHK(hipEventRecord(e0, s));
 	int levels = 0, rc = SP_OK;
-	for (int i = 0; i < n && !rc; i++) rc = adjoint_sweeps_image(imgs[i], P, s, &levels);
-	// a wait that gave up left wrong values
-	(void)hipMemcpyAsync(g_as_err->h_gs_err, g_as_err->gs_err, sizeof(int),
-			hipMemcpyDeviceToHost, s);
+	bool timed_out = false;   // a wait gave up and left wrong values
+	for (int i = 0; i < n && !rc; i++)
+		rc = adjoint_sweeps_image(imgs[i], P, s, &levels, &timed_out);
 	(void)hipEventRecord(e1, s);
+	if (g_as) timed_out |= as_timed_out(*g_as, s);
 	if (hipEventSynchronize(e1) != hipSuccess && !rc)
 		rc = set_err(SP_ERR_HIP, "gradient of the sweeps failed");
 	float ms = 0;
 	(void)hipEventElapsedTime(&ms, e0, e1);
 	(void)hipEventDestroy(e0);
 	(void)hipEventDestroy(e1);
-	if (*g_as_err->h_gs_err) {
-		*g_as_err->h_gs_err = 0;
-		(void)hipMemset(g_as_err->gs_err, 0, sizeof(int));
-		if (!rc) rc = set_err(SP_ERR_HIP, "dependence wait timed out in the gradient of "
-				"the sweeps");
-	}
+	if (timed_out && !rc)
+		rc = set_err(SP_ERR_HIP, "dependence wait timed out in the gradient of the sweeps");
 	TRY(rc);
 	if (st) { st->levels = levels; st->cg_iters_finest = 0; st->elapsed_ms = ms; }
 	return SP_OK;
