@@ -2977,16 +2977,22 @@ extern "C" int sp_amle_device(float *d_out, const float *d_in, const float *d_in
 	AmlePlan *A = g_amle;
 	// a dependence wait of an earlier call that timed out (the calls are
 	// asynchronous: it is reported by the next call, once that work is done)
-	if (A && A->used && A->mem.gs_flow_used && hipEventQuery(A->done) == hipSuccess
-			&& *A->mem.h_gs_err) {
+	auto timed_out = [&] {
+		if (!A || !A->used || !A->mem.gs_flow_used || hipEventQuery(A->done) != hipSuccess
+				|| !*A->mem.h_gs_err)
+			return false;
 		*A->mem.h_gs_err = 0;
 		(void)hipMemset(A->mem.gs_err, 0, sizeof(int));
-		return set_err(SP_ERR_HIP, "AMLE tile dependence wait timed out in an earlier call");
-	}
+		return true;
+	};
+	const char *const late = "AMLE tile dependence wait timed out in an earlier call";
+	if (timed_out()) return set_err(SP_ERR_HIP, "%s", late);
 	if (!A || A->w != w || A->h != h || A->pd != pd || A->nn != nn ||
 			A->niter != niter || A->trace != trace || A->var != var || A->stream != streams) {
-		// the old plan's scratch may still be in use on its stream
+		// the old plan's scratch may still be in use on its stream, and its
+		// error word goes with it
 		if (A && A->used) HIPCHK(hipEventSynchronize(A->done));
+		if (timed_out()) return set_err(SP_ERR_HIP, "%s", late);
 		const size_t n = (size_t)w * h * pd;
 		int rc = SP_OK;
 		for (bool stream = true;; stream = false) {
