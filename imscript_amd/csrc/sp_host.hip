@@ -2945,6 +2945,19 @@ static int amle_args(const float *out, const float *in, int w, int h, int pd,
 
 static std::mutex g_amle_mu;
 static AmlePlan *g_amle = nullptr;
+
+// whether a dependence wait of the plan's last call, once that is done, gave
+// up; the word is cleared
+static bool amle_timed_out(AmlePlan *A)
+{
+	if (!A || !A->used || !A->mem.gs_flow_used || hipEventQuery(A->done) != hipSuccess
+			|| !*A->mem.h_gs_err)
+		return false;
+	*A->mem.h_gs_err = 0;
+	(void)hipMemset(A->mem.gs_err, 0, sizeof(int));
+	return true;
+}
+
 static int amle_run(AmlePlan &A, float *d_out, const float *d_in, const float *d_init,
 		hipStream_t s);
 
@@ -2977,22 +2990,14 @@ extern "C" int sp_amle_device(float *d_out, const float *d_in, const float *d_in
 	AmlePlan *A = g_amle;
 	// a dependence wait of an earlier call that timed out (the calls are
 	// asynchronous: it is reported by the next call, once that work is done)
-	auto timed_out = [&] {
-		if (!A || !A->used || !A->mem.gs_flow_used || hipEventQuery(A->done) != hipSuccess
-				|| !*A->mem.h_gs_err)
-			return false;
-		*A->mem.h_gs_err = 0;
-		(void)hipMemset(A->mem.gs_err, 0, sizeof(int));
-		return true;
-	};
 	const char *const late = "AMLE tile dependence wait timed out in an earlier call";
-	if (timed_out()) return set_err(SP_ERR_HIP, "%s", late);
+	if (amle_timed_out(A)) return set_err(SP_ERR_HIP, "%s", late);
 	if (!A || A->w != w || A->h != h || A->pd != pd || A->nn != nn ||
 			A->niter != niter || A->trace != trace || A->var != var || A->stream != streams) {
 		// the old plan's scratch may still be in use on its stream, and its
 		// error word goes with it
 		if (A && A->used) HIPCHK(hipEventSynchronize(A->done));
-		if (timed_out()) return set_err(SP_ERR_HIP, "%s", late);
+		if (amle_timed_out(A)) return set_err(SP_ERR_HIP, "%s", late);
 		const size_t n = (size_t)w * h * pd;
 		int rc = SP_OK;
 		for (bool stream = true;; stream = false) {
@@ -3091,6 +3096,10 @@ extern "C" int sp_amle_host(float *out, const float *in, const float *init,
 	}
 	TRY(sp_amle_device(d_out, d_in, d_init, w, h, pd, nn, niter, trace, nullptr));
 	HIPCHK(hipMemcpy(out, d_out, n * 4, hipMemcpyDeviceToHost));
+	// (the copy has waited for the sweeps: their error is this call's)
+	std::lock_guard<std::mutex> lk(g_amle_mu);
+	if (amle_timed_out(g_amle))
+		return set_err(SP_ERR_HIP, "AMLE tile dependence wait timed out");
 	return SP_OK;
 }
 

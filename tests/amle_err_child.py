@@ -1,7 +1,8 @@
 """Child process of the GPU test of AMLE's error path: with
 SIMPOIS_HIP_GS_FLOW_SPIN=0 the sweeps of a large plane give up a dependence
 wait, and the next call reports it also where it comes at once, with another
-size that replaces the kept plan.  Exit status 0 when it did."""
+size that replaces the kept plan; a call on host arrays reports its own.  Exit
+status 0 when they did."""
 import os
 import sys
 
@@ -29,6 +30,15 @@ def main():
             return 1
     m.amle(small, 4, 1)      # reported once
     torch.cuda.synchronize()
+    try:                     # host arrays: the call is not asynchronous
+        m.amle(x.cpu().numpy(), 4, 200)
+        print("host arrays: no error", flush=True)
+        return 1
+    except Exception as e:
+        print(f"host arrays: {type(e).__name__}: {e}", flush=True)
+        if "dependence wait" not in str(e):
+            return 1
+    m.amle(small.cpu().numpy(), 4, 1)
     return 0
 
 
