@@ -769,7 +769,7 @@ def run_amle(a):
                                    if not gs_flow() else
                                    "k_ss_run (streaming bands of 64 skewed rows, all "
                                    "sweeps in one launch)" if nn == 4
-                                   and "SIMPOIS_HIP_AMLE_VARIANT" not in os.environ else
+                                   and not os.environ.get("SIMPOIS_HIP_AMLE_VARIANT") else
                                    f"k_amle_flow<{'4-neighbour' if nn == 4 else 'table'}> "
                                    f"(tile {shape} = BIxBJxBT: BT raster sweeps fused per "
                                    "pass; one launch per pass, each skewed tile started "
